@@ -366,11 +366,10 @@ int wake_domain_set_wall_temperature(wake_domain* d, int x0, int y0, int x1, int
 /* work-group width along x for the step kernel (64, 128, 192, 256; 0 = auto) */
 int wake_domain_set_block_x(wake_domain* d, int block_x);
 /* Extension (no reference counterpart): on = 1 (default) lets
- * wake_domain_run take 8 steps per launch on a fully periodic 2D domain
- * whose cells are all Fluid, with no inlet, outlet, force probe or
- * temperature, of up to 2^21 nodes (FP32) or 2^17 (16-bit storage), where
- * single launches are bound by the launch rate; the result is the same as
- * 8 single steps.  0 keeps one launch per step. */
+ * wake_domain_run take up to 8 steps per launch on 2D domains without curved
+ * links and without the convective outlet (16-bit storage: up to 2^23 nodes,
+ * 2^19 with temperature; not BF16 temperature domains, not timed runs), with
+ * the same result; 0: one launch per step. */
 int wake_domain_set_multistep(wake_domain* d, int on);
 /* FP16 / BF16 storage: 1 (default) addresses the populations through a
  * buffer descriptor when the buffer is under 4 GiB; 0 always through 64-bit

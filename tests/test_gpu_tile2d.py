@@ -1,0 +1,132 @@
+"""Bounded 2D domains run up to 8 steps per launch from LDS tiles
+(tile2d.hpp).  Every node update is the single-step kernel's, so a run must
+give the same bits as the same number of single steps: walls, obstacles, a
+moving wall, parabolic and noisy inlets, the pressure outlet, solid nodes in
+periodic streaming, the temperature coupling and the force history, at sizes
+around the tiles' own extent and their halo, and when runs of every length
+alternate with single steps, force reads and geometry changes.
+"""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+SIZES = [(240, 80), (64, 33), (33, 17), (16, 16), (17, 48), (9, 5), (131, 8)]
+
+
+@pytest.fixture(scope="module")
+def wa():
+    import wake_amd
+
+    if wake_amd._lib.lib().wake_hip_device_count() <= 0:
+        pytest.fail("no GPU visible to the HIP runtime")
+    return wake_amd
+
+
+def _start(g, nx, ny, seed=3):
+    r = np.random.default_rng(seed)
+    u = r.uniform(-0.02, 0.02, (2, nx * ny)).astype(np.float32)
+    g.initialize_fields(np.ones(nx * ny, np.float32), u[0] + np.float32(0.03), u[1])
+
+
+def _channel(wa, nx, ny, storage, turb=False):
+    g = wa.LatticeGrid2D(nx, ny, 0.6, storage=storage)
+    _start(g, nx, ny)
+    g.set_les_coupled(True)
+    g.set_inflow_parabolic(0.05)
+    if turb:
+        g.set_inflow_turbulence(0.05, 11)
+    g.set_outflow_east(1.0)
+    g.set_solid_box(0, 0, nx - 1, 0)
+    g.set_solid_box(0, ny - 1, nx - 1, ny - 1)
+    g.set_solid_circle(nx / 3.0, ny / 2.0, max(1.0, ny / 8.0))
+    return g
+
+
+def _lid(wa, nx, ny, storage, periodic_y=False):
+    g = wa.LatticeGrid2D(nx, ny, 0.58, storage=storage)
+    _start(g, nx, ny, 5)
+    g.set_solid_box(0, 0, 0, ny - 1)
+    g.set_solid_box(nx // 2, ny // 3, nx // 2 + 1, ny // 2)
+    g.set_moving_wall_north(0.06)
+    if periodic_y:
+        g.set_periodic_axes(True, False)
+    return g
+
+
+def _solid_in_periodic(wa, nx, ny, storage):
+    g = wa.LatticeGrid2D(nx, ny, 0.7, storage=storage)
+    _start(g, nx, ny, 9)
+    g.set_solid_box(1, 1, 2, 2)
+    g.set_periodic(True)
+    return g
+
+
+def _cavity(wa, nx, ny, storage):
+    g = wa.LatticeGrid2D(nx, ny, 0.58, storage=storage)
+    g.initialize(1.0, 0.0, 0.0)
+    for box in ((0, 0, nx - 1, 0), (0, ny - 1, nx - 1, ny - 1), (0, 0, 0, ny - 1), (nx - 1, 0, nx - 1, ny - 1)):
+        g.set_solid_box(*box)
+    g.enable_thermal(0.62, 1e-3, 0.5, 0.5)
+    g.set_temperature_field(np.random.default_rng(1).uniform(0, 1, nx * ny).astype(np.float32))
+    g.set_wall_temperature(0, 0, 0, ny - 1, 1.0)
+    return g
+
+
+SCENES = {
+    "channel": (_channel, [("TRT", False), ("MRT", True), ("BGK", False), ("TRT", True)], True),
+    "noisy": (lambda *a: _channel(*a, turb=True), [("BGK", True)], True),
+    "lid": (_lid, [("BGK", False), ("TRT", True)], True),
+    "lid_periodic_y": (lambda *a: _lid(*a, periodic_y=True), [("MRT", False)], True),
+    "solid_periodic": (_solid_in_periodic, [("MRT", False)], False),
+    "cavity": (_cavity, [("MRT", False), ("BGK", False)], None),
+}
+
+
+def _state(g, thermal):
+    out = [g.f_src_data().copy(), g.rho_data(), g.ux_data(), g.uy_data()]
+    return out + ([g.temperature_data()] if thermal else [])
+
+
+@pytest.mark.parametrize("storage", [0, 1, 2])
+@pytest.mark.parametrize("scene", list(SCENES))
+@pytest.mark.parametrize("nx,ny", SIZES)
+def test_tile_run_equals_single_steps(wa, nx, ny, scene, storage):
+    make, kinds, forces = SCENES[scene]
+    for coll, les, gx, gy in [k + g for k in kinds for g in ((1e-6, -2e-6), (0.0, 0.0))]:
+        ends = []
+        for multi in (True, False):
+            g = make(wa, nx, ny, storage)
+            g.set_multistep(multi)
+            if forces:
+                g.set_force_probe(nx / 3.0, ny / 2.0, 0.0, 0.0)
+            for steps in (1, 3, 8, 2, 21):  # from a materialised state, remainders, several launches
+                g.run(steps, coll, gx=gx, gy=gy, use_les=les, smag=0.17)
+            end = _state(g, forces is None)
+            if forces:
+                end.append(g.force_history()[1])
+                assert end[-1].shape == (36, 3)
+            ends.append(end)
+        for a, b in zip(*ends):
+            assert np.array_equal(a, b, equal_nan=True), (coll, les, gx)
+
+
+def test_force_history_over_mixed_steps(wa):
+    """Tile launches, single steps, reads, a ring's worth of steps and a
+    geometry change between them leave the history of single steps."""
+    hist = []
+    for multi in (True, False):
+        g = _channel(wa, 150, 50, 0)
+        g.set_multistep(multi)
+        g.set_force_probe(50.0, 25.0, 0.0, 20.0)
+        g.run(70, "MRT", use_les=True, smag=0.17)
+        g.step("MRT", use_les=True, smag_const=0.17)
+        g.run(9, "MRT", use_les=True, smag=0.17)
+        mid = g.force_history()[1].copy()
+        g.run(5, "MRT", use_les=True, smag=0.17)
+        g.set_solid_box(90, 20, 92, 24)
+        g.run(130, "MRT", use_les=True, smag=0.17)
+        first, f = g.force_history()
+        assert first == 0 and f.shape == (216, 3) and np.array_equal(f[:81], mid)
+        hist.append(f)
+    assert np.array_equal(*hist)

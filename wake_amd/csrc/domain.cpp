@@ -744,34 +744,57 @@ void Domain::materialize() {
 }
 
 // ------------------------------------------------------------------ step
-bool Domain::tb_eligible() {
-  if (dim_ != 2 || lattice_ != 9 || thermal_ || probe_ || s_buf_ >= 0 || !all_fluid_ || !tb_enabled_) return false;
-  // Only where single-step launches are bound by the launch rate: measured,
-  // 8 steps per launch reach about 75 G node-steps/s (the tile loads and
-  // the 2.15x redundant halo updates bound it), while single steps of larger
-  // domains run at the HBM rate (FP32: 58.5k vs 71.3k MLUPS at 1024^2,
-  // 82.8k vs 77.5k at 4096^2; FP16: 92.3k vs 65.2k at 1024^2).
-  if (N_ > (storage_ == kStoreF32 ? (1u << 21) : (1u << 17))) return false;
-  const StepArgs a = args(true);
-  return a.periodic_mode && !a.inflow && !a.outflow;
+bool Domain::tile_eligible() const {
+  if (dim_ != 2 || !tile_enabled_) return false;
+  // curved links and the convective outlet read past the tile's halo
+  if (n_bfl_nodes_ > 0 || outflow_ == 2) return false;
+  // (the temperature kernels with BF16 storage round some products otherwise
+  // in a step loop than in a single step)
+  if (thermal_ && storage_ == kStoreBF16) return false;
+  // Measured, us a step of single launches / tiles: FP32 channels 4.4 / 1.7 at
+  // 240 x 80, 13.2 / 8.3 at 1500 x 403, 202 / 147 at 4096^2; FP32 temperature
+  // 6.1 / 2.1 at 240 x 80, 36 / 31 at 1536 x 1024, 341 / 326 at 4096^2.  With
+  // 16-bit storage a single launch moves half the bytes, so the largest
+  // domains do without: TRT channels 19.2 / 19.7 at 1536 x 1024, 151 / 153 at
+  // 4096^2 (MRT 135 / 130); temperature 14.3 / 13.7 at 1024 x 512, 30 / 37 at
+  // 1536 x 1024.
+  if (storage_ == kStoreF32) return true;
+  return N_ <= (thermal_ ? 1u << 19 : 1u << 23);
 }
 
-void Domain::step_tb(int collision, float gx, float gy, bool use_les, float smag) {
-  version_ += kTbSteps;
+bool Domain::plain_periodic() const {
+  return all_fluid_ && is_periodic_ && !has_moving_wall_ && !has_inflow_ && outflow_ == 0 && !thermal_;
+}
+
+void Domain::step_tile(int nsteps, int collision, float gx, float gy, bool use_les, float smag) {
+  version_ += static_cast<uint64_t>(nsteps);
+  const bool from_s = s_buf_ >= 0;
+  TileForces mf{};
+  if (probe_) {
+    probe_sync();
+    // a launch from a materialised S forms S_{k+1} first
+    if (from_s) probe_sample_current();
+    mf = probe_tile(nsteps);
+  }
   StepArgs a = args(true);
   a.tau = tau_;
   a.gx = gx;
   a.gy = gy;
   a.gz = 0.0f;
   a.cs = smag;
-  const int out = 1 - a_buf_;
-  check(launch_step_tb(lattice_, storage_, collision, use_les && les_coupled_, a, buf_[a_buf_], buf_[out], stream_),
-        "periodic step");
+  for (int k = 0; k < 3; ++k) a.mem_c[k] = probe_c_[k];
+  a.mem_rmax = probe_rmax_;
+  const int in = from_s ? s_buf_ : a_buf_, out = 1 - in;
+  check(launch_tile2d(storage_, collision, use_les && les_coupled_, thermal_, from_s, !plain_periodic() || mf.index, nsteps, a,
+                      buf_[in], buf_[out], gbuf_[in], gbuf_[out], mf, stream_),
+        "tile steps");
   a_buf_ = out;
+  s_buf_ = -1;
   g_last_[0] = gx;
   g_last_[1] = gy;
   g_last_[2] = 0.0f;
-  step_count_ += kTbSteps;
+  step_count_ += static_cast<uint64_t>(nsteps);
+  if (probe_) fh_next_ = tile_end_ = step_count_;
   invalidate_mirrors();
 }
 
@@ -860,10 +883,15 @@ float Domain::run(int steps, int collision, float gx, float gy, float gz, bool u
   timed_launches_ = 0;
   try {
     int s = 0;
-    // fully periodic D2Q9 without special nodes: kTbSteps steps per launch
-    // (an untimed run only: the kernel timer samples single-step launches)
-    if (!timed && steps >= kTbSteps && tb_eligible()) {
-      for (; steps - s >= kTbSteps; s += kTbSteps) step_tb(collision, gx, gy, use_les, smag);
+    // 2D domains: up to kTbSteps steps per launch (an untimed run only: the
+    // kernel timer samples single-step launches)
+    if (!timed && tile_eligible()) {
+      const int most = tile2d_steps_of(nx_, ny_, thermal_ && storage_ == kStoreF32);
+      while (steps - s >= 2) {
+        const int k = std::min(steps - s, most);
+        step_tile(k, collision, gx, gy, use_les, smag);
+        s += k;
+      }
     }
     for (; s < steps; ++s) step(collision, gx, gy, gz, use_les, smag);
   } catch (...) {
@@ -1092,6 +1120,33 @@ Domain::MemRows Domain::build_mem_rows(float ccx, float ccy, float ccz, float r_
   return r;
 }
 
+// Per-row counts, their prefix on the host, then the nodes.
+int* Domain::build_mem_nodes(const MemRows& rows, float ccx, float ccy, float ccz, float r_max, int* count) {
+  *count = 0;
+  const int nr = rows.nrows;
+  if (nr == 0) return nullptr;
+  StepArgs a = args(false);
+  a.mem_c[0] = ccx;
+  a.mem_c[1] = ccy;
+  a.mem_c[2] = ccz;
+  a.mem_rmax = r_max;
+  int* d_cnt = static_cast<int*>(alloc(2 * static_cast<size_t>(nr) * sizeof(int)));
+  check(launch_mem_row_nodes(lattice_, a, rows.d_list, nr, d_cnt, nullptr, nullptr, stream_), "link nodes");
+  std::vector<int> cnt(nr), off(nr);
+  check(hipMemcpyAsync(cnt.data(), d_cnt, nr * sizeof(int), hipMemcpyDeviceToHost, stream_), "link nodes");
+  check(hipStreamSynchronize(stream_), "link nodes");
+  for (int r = 0; r < nr; ++r) {
+    off[r] = *count;
+    *count += cnt[r];
+  }
+  int* d_nodes = static_cast<int*>(alloc(std::max(1, *count) * sizeof(int)));
+  check(hipMemcpyAsync(d_cnt + nr, off.data(), nr * sizeof(int), hipMemcpyHostToDevice, stream_), "link nodes");
+  check(launch_mem_row_nodes(lattice_, a, rows.d_list, nr, d_cnt, d_cnt + nr, d_nodes, stream_), "link nodes");
+  check(hipStreamSynchronize(stream_), "link nodes");
+  release(d_cnt);
+  return d_nodes;
+}
+
 void Domain::free_mem_rows(MemRows& r) {
   if (r.d_rows || r.d_list) check(hipStreamSynchronize(stream_), "free rows");
   release(r.d_rows);
@@ -1174,13 +1229,17 @@ long long Domain::count_nonfinite(long long* first) {
 // ------------------------------------------------------------- force probe
 void Domain::set_force_probe(float ccx, float ccy, float ccz, float r_max) {
   if (thermal_) throw HipError("the force history is not available on temperature-coupled domains");
+  // the linked rows and nodes belong to the centre, the radius and the
+  // geometry (probe_epoch_): a restart of the same probe keeps them
+  if (!probe_ || probe_c_[0] != ccx || probe_c_[1] != ccy || probe_c_[2] != ccz || probe_rmax_ != r_max) {
+    if (probe_rows_.d_rows) free_mem_rows(probe_rows_);
+    probe_epoch_ = tile_epoch_ = ~0ull;
+  }
   probe_ = true;
   probe_c_[0] = ccx;
   probe_c_[1] = ccy;
   probe_c_[2] = ccz;
   probe_rmax_ = r_max;
-  if (probe_rows_.d_rows) free_mem_rows(probe_rows_);
-  probe_epoch_ = ~0ull;
   if (!d_fhist_) d_fhist_ = static_cast<double*>(alloc(3 * static_cast<size_t>(kForceHistCap) * sizeof(double)));
   probe_restart();
 }
@@ -1188,12 +1247,13 @@ void Domain::set_force_probe(float ccx, float ccy, float ccz, float r_max) {
 void Domain::clear_force_probe() {
   probe_ = false;
   if (probe_rows_.d_rows) free_mem_rows(probe_rows_);
-  probe_epoch_ = ~0ull;
+  probe_epoch_ = tile_epoch_ = ~0ull;
   h_fhist_.clear();
 }
 
 void Domain::probe_restart() {
   fh_first_ = fh_next_ = fh_folded_ = fh_dbase_ = fh_host_ = step_count_;
+  tile_first_ = tile_end_ = step_count_;
   h_fhist_.clear();
 }
 
@@ -1220,6 +1280,7 @@ void Domain::probe_sync() {
 
 void Domain::probe_fold(uint64_t upto) {
   if (upto <= fh_folded_) return;
+  probe_flush_tiles();
   if (upto - fh_dbase_ > static_cast<uint64_t>(kForceHistCap)) {
     // the device history is full: move what is folded to the host
     const size_t n = static_cast<size_t>(fh_folded_ - fh_host_);
@@ -1242,6 +1303,45 @@ void Domain::probe_fold(uint64_t upto) {
 double* Domain::probe_slot(uint64_t k) {
   if (k - fh_folded_ >= static_cast<uint64_t>(kForceRing)) probe_fold(k);
   return d_ring_ + 3 * static_cast<size_t>(std::max(1, probe_rows_.nslots)) * (k % kForceRing);
+}
+
+// Samples a tile launch of nsteps steps from step_count_ takes: S_{fh_next_}
+// up to S_{step_count_ + nsteps - 1}, as per-node sums in d_fnode_ until
+// probe_flush_tiles() turns them into the ring's partials.
+TileForces Domain::probe_tile(int nsteps) {
+  if (tile_end_ != fh_next_) {
+    probe_flush_tiles();
+    tile_first_ = tile_end_ = fh_next_;
+  }
+  if (step_count_ + nsteps - fh_folded_ > static_cast<uint64_t>(kForceRing)) probe_fold(fh_next_);
+  if (tile_epoch_ != probe_epoch_) {
+    if (d_findex_ || d_fnode_) check(hipStreamSynchronize(stream_), "force nodes");
+    release(d_findex_);
+    release(d_fnode_);
+    d_findex_ = nullptr;
+    d_fnode_ = nullptr;
+    int* d_nodes =
+        build_mem_nodes(probe_rows_, probe_c_[0], probe_c_[1], probe_c_[2], probe_rmax_, &n_fnodes_);
+    if (n_fnodes_ > 0) {
+      d_findex_ = static_cast<int*>(alloc(N_ * sizeof(int)));
+      d_fnode_ = static_cast<double*>(alloc(3 * sizeof(double) * kForceRing * static_cast<size_t>(n_fnodes_)));
+      check(hipMemsetAsync(d_findex_, 0xff, N_ * sizeof(int), stream_), "force nodes");
+      check(launch_index_nodes(d_nodes, n_fnodes_, d_findex_, stream_), "force nodes");
+      check(hipStreamSynchronize(stream_), "force nodes");
+    }
+    release(d_nodes);
+    tile_epoch_ = probe_epoch_;
+  }
+  return TileForces{d_findex_, d_fnode_, n_fnodes_, kForceRing};
+}
+
+void Domain::probe_flush_tiles() {
+  if (tile_first_ < tile_end_ && n_fnodes_ > 0)
+    check(launch_mem_slots(TileForces{d_findex_, d_fnode_, n_fnodes_, kForceRing}, probe_rows_.d_list,
+                           probe_rows_.nrows, nx_, static_cast<long long>(tile_first_),
+                           static_cast<int>(tile_end_ - tile_first_), d_ring_, stream_),
+          "force partials");
+  tile_first_ = tile_end_;
 }
 
 // The sample of S_{step_count_} when no launch has formed it yet: read from
@@ -1371,32 +1471,7 @@ const int* Domain::batch_mem_nodes(float ccx, float ccy, float ccz, float r_max,
     }
     batch_rows_ = build_mem_rows(ccx, ccy, ccz, r_max);
     batch_rows_key_ = key;
-    n_batch_nodes_ = 0;
-    const int nr = batch_rows_.nrows;
-    if (nr > 0) {
-      StepArgs a = args(false);
-      a.mem_c[0] = ccx;
-      a.mem_c[1] = ccy;
-      a.mem_c[2] = ccz;
-      a.mem_rmax = r_max;
-      // per-row counts, their prefix on the host, then the nodes
-      int* d_cnt = static_cast<int*>(alloc(2 * static_cast<size_t>(nr) * sizeof(int)));
-      check(launch_mem_row_nodes(lattice_, a, batch_rows_.d_list, nr, d_cnt, nullptr, nullptr, stream_),
-            "batch nodes");
-      std::vector<int> cnt(nr), off(nr);
-      check(hipMemcpyAsync(cnt.data(), d_cnt, nr * sizeof(int), hipMemcpyDeviceToHost, stream_), "batch nodes");
-      check(hipStreamSynchronize(stream_), "batch nodes");
-      for (int r = 0; r < nr; ++r) {
-        off[r] = n_batch_nodes_;
-        n_batch_nodes_ += cnt[r];
-      }
-      d_batch_nodes_ = static_cast<int*>(alloc(std::max(1, n_batch_nodes_) * sizeof(int)));
-      check(hipMemcpyAsync(d_cnt + nr, off.data(), nr * sizeof(int), hipMemcpyHostToDevice, stream_), "batch nodes");
-      check(launch_mem_row_nodes(lattice_, a, batch_rows_.d_list, nr, d_cnt, d_cnt + nr, d_batch_nodes_, stream_),
-            "batch nodes");
-      check(hipStreamSynchronize(stream_), "batch nodes");
-      release(d_cnt);
-    }
+    d_batch_nodes_ = build_mem_nodes(batch_rows_, ccx, ccy, ccz, r_max, &n_batch_nodes_);
   }
   *count = n_batch_nodes_;
   return d_batch_nodes_;

@@ -90,9 +90,9 @@ class Domain {
 
   // --- stepping
   void step(int collision, float gx, float gy, float gz, bool use_les, float smag);
-  // run() takes kTbSteps steps per launch where tb_eligible() (fully periodic
-  // D2Q9 without special nodes, no force probe); off: one launch per step.
-  void set_multistep(bool on) { tb_enabled_ = on; }
+  // run() takes up to kTbSteps steps per launch where tile_eligible() (2D
+  // domains); off: one launch per step.
+  void set_multistep(bool on) { tile_enabled_ = on; }
   // `steps` steps; returns the device time in ms measured with events on the
   // domain's stream around the launches.
   float run(int steps, int collision, float gx, float gy, float gz, bool use_les, float smag, bool timed);
@@ -230,6 +230,8 @@ class Domain {
     int nslots = 0;
   };
   MemRows build_mem_rows(float cx, float cy, float cz, float r_max);
+  // The nodes of those rows holding links, in node order (a device list).
+  int* build_mem_nodes(const MemRows& rows, float cx, float cy, float cz, float r_max, int* count);
   void free_mem_rows(MemRows& r);
   const MemRows& cached_mem_rows(float cx, float cy, float cz, float r_max);
   StepArgs with_mem(StepArgs a, const MemRows& r, double* part, const float c[3], float r_max) const;
@@ -237,6 +239,8 @@ class Domain {
   void probe_fold(uint64_t upto);   // fold the samples of steps [fh_folded_, upto)
   void probe_sample_current();      // sample S_{step_count_} if no launch has
   double* probe_slot(uint64_t k);   // ring entry of step k (folding first if it is taken)
+  TileForces probe_tile(int nsteps);  // where the next tile launch writes its samples
+  void probe_flush_tiles();         // partials of the samples tile launches left
   void probe_restart();
 
   int dim_, lattice_, Q_, nx_, ny_, nz_;
@@ -280,10 +284,11 @@ class Domain {
   uint8_t* d_flags_ = nullptr;
   uint8_t* d_cls_ = nullptr;
   uint32_t* d_bmask_ = nullptr;  // per node: bounce mask of the kClsSlow nodes
-  bool tb_eligible();
-  void step_tb(int collision, float gx, float gy, bool use_les, float smag);
+  bool tile_eligible() const;
+  bool plain_periodic() const;   // no node carries a class bit
   bool all_fluid_ = false;       // every cell type Fluid (set with the class bytes)
-  bool tb_enabled_ = true;       // run() may take kTbSteps steps per launch
+  void step_tile(int nsteps, int collision, float gx, float gy, bool use_les, float smag);
+  bool tile_enabled_ = true;     // run() may take up to kTbSteps steps per launch
   int* d_aux_ = nullptr;
   BflNode* d_bfl_ = nullptr;
   int* d_bfl_nodes_ = nullptr;
@@ -317,6 +322,13 @@ class Domain {
   float probe_rmax_ = 0.0f;
   MemRows probe_rows_;
   uint64_t probe_epoch_ = ~0ull;
+  // samples of tile launches: per-node sums (a ring of kForceRing steps),
+  // the place of each node in them, and the steps not yet in d_ring_
+  uint64_t tile_epoch_ = ~0ull;
+  int* d_findex_ = nullptr;
+  double* d_fnode_ = nullptr;
+  int n_fnodes_ = 0;
+  uint64_t tile_first_ = 0, tile_end_ = 0;
   double* d_ring_ = nullptr;
   size_t ring_cap_ = 0;  // in doubles
   double* d_fhist_ = nullptr;

@@ -107,13 +107,36 @@ inline int mem_waves_per_row(int nx) { return (nx + 63) / 64; }
 
 // Launchers (step_kernels.hip).  `lattice` is 9, 19 or 27.
 hipError_t launch_build_class(int lattice, const StepArgs& a, uint8_t* cls, uint32_t* bmask, hipStream_t s);
-// Steps per launch of the fully periodic D2Q9 path (launch_step_tb).
+// Most steps of one tile launch (launch_tile2d): the halo of its LDS tiles.
 inline constexpr int kTbSteps = 8;
-// kTbSteps pull + collide steps of a fully periodic D2Q9 domain whose class
-// bytes are all zero (no solid, inlet or outlet node), A_{k-1} in `in` to
-// A_{k-1+kTbSteps} in `out`.
-hipError_t launch_step_tb(int lattice, int storage, int collision, bool les, const StepArgs& a, const void* in,
-                          void* out, hipStream_t s);
+// Where a tile launch writes the force sums (3 doubles) of the nodes holding
+// momentum-exchange links: node n's sum of step k goes to
+// out[3 ((k % ring) count + index[n]) ..]; index[n] is -1 for other nodes.
+// index null: no forces.
+struct TileForces {
+  const int* index;
+  double* out;
+  int count;
+  int ring;
+};
+// Steps a tile launch of such a domain takes best (at most kTbSteps);
+// one_per_unit: a compute unit holds one of its tiles (FP32 temperature).
+int tile2d_steps_of(int nx, int ny, bool one_per_unit);
+// nsteps (at most kTbSteps) steps of a 2D domain without curved links and
+// without the convective outlet, from A_{k-1} in `in` (from_s: from a
+// materialised S_k, the first step collides only) to A_{k-1+nsteps} in `out`;
+// edges: false only when every class byte is zero and mf takes nothing;
+// gin / gout: the temperature populations of a thermal domain (tile2d.hip;
+// not with BF16 storage).
+hipError_t launch_tile2d(int storage, int collision, bool les, bool thermal, bool from_s, bool edges, int nsteps,
+                         const StepArgs& a, const void* in, void* out, const float* gin, float* gout,
+                         const TileForces& mf, hipStream_t s);
+// The per-wave partials (the layout of a single-step launch's mem_part, ring
+// of mf.ring steps) of steps first .. first + count - 1 from those sums.
+hipError_t launch_mem_slots(const TileForces& mf, const int* row_list, int nrows, int nx, long long first, int count,
+                            double* ring, hipStream_t s);
+// index[nodes[i]] = i.
+hipError_t launch_index_nodes(const int* nodes, int count, int* index, hipStream_t s);
 hipError_t launch_mark_bfl(const int* nodes, int count, uint8_t* cls, int* aux, hipStream_t s);
 // pull=false: collide-only from the materialised S state.  block_x is the
 // work-group width along x (64, 128 or 256).

@@ -82,10 +82,16 @@ __device__ __forceinline__ void density_momentum(const float (&f)[L::Q], float& 
 }
 
 // Velocity with the Guo half-force shift (d3q19_moments.ispc:60-64).
-template <bool FAST = false>
+template <bool FAST = false, bool FORCE = true>
 __device__ __forceinline__ void guo_velocity(float rho, float jx, float jy, float jz, float gx, float gy, float gz,
                                              float& ux, float& uy, float& uz) {
   const float inv_rho = recip<FAST>(rho);
+  if constexpr (!FORCE) {
+    ux = jx * inv_rho;
+    uy = jy * inv_rho;
+    uz = jz * inv_rho;
+    return;
+  }
   ux = (jx + 0.5f * rho * gx) * inv_rho;
   uy = (jy + 0.5f * rho * gy) * inv_rho;
   uz = (jz + 0.5f * rho * gz) * inv_rho;
@@ -187,16 +193,18 @@ struct Macro {
   float rho, ux, uy, uz;
 };
 
+// The collisions below take FORCE = false where the body force is zero: its
+// terms, all exact zeros, are not formed (the same values).
+
 // BGK with Guo forcing, in place (d3q19_collision_bgk.ispc:4-75,
-// d2q9_collision_bgk.ispc:5-86).
-template <class L, bool FAST = false>
-__device__ __forceinline__ Macro collide_bgk(float (&f)[L::Q], float tau, float gx, float gy, float gz) {
-  const float omega = recip<FAST>(tau);
+// d2q9_collision_bgk.ispc:5-86), omega = 1 / tau.
+template <class L, bool FAST = false, bool FORCE = true>
+__device__ __forceinline__ Macro collide_bgk_rate(float (&f)[L::Q], float omega, float gx, float gy, float gz) {
   const float pre = 1.0f - 0.5f * omega;
   float rho, jx, jy, jz, ux, uy, uz;
   density_momentum<L>(f, rho, jx, jy, jz);
-  guo_velocity<FAST>(rho, jx, jy, jz, gx, gy, gz, ux, uy, uz);
-  const float u_dot_g = ux * gx + uy * gy + uz * gz;
+  guo_velocity<FAST, FORCE>(rho, jx, jy, jz, gx, gy, gz, ux, uy, uz);
+  const float u_dot_g = FORCE ? ux * gx + uy * gy + uz * gz : 0.0f;
   const float usq = ux * ux + uy * uy + uz * uz;
   static_for<L::Q>([&](auto qc) {
     constexpr int q = decltype(qc)::value;
@@ -204,9 +212,14 @@ __device__ __forceinline__ Macro collide_bgk(float (&f)[L::Q], float tau, float 
     const float cg = cdot<L, q>(gx, gy, gz);
     const float fe = L::w[q] * rho * (1.0f + 3.0f * cu + 4.5f * cu * cu - 1.5f * usq);
     const float Fi = pre * L::w[q] * rho * (3.0f * (cg - u_dot_g) + 9.0f * cu * cg);
-    f[q] = f[q] - omega * (f[q] - fe) + Fi;
+    if constexpr (FORCE) f[q] = f[q] - omega * (f[q] - fe) + Fi;
+    else f[q] = f[q] - omega * (f[q] - fe);
   });
   return {rho, ux, uy, uz};
+}
+template <class L, bool FAST = false>
+__device__ __forceinline__ Macro collide_bgk(float (&f)[L::Q], float tau, float gx, float gy, float gz) {
+  return collide_bgk_rate<L, FAST>(f, recip<FAST>(tau), gx, gy, gz);
 }
 
 // TRT with split Guo forcing, in place (d3q19_collision_trt.ispc:5-93,
@@ -215,15 +228,14 @@ __device__ __forceinline__ Macro collide_bgk(float (&f)[L::Q], float tau, float 
 // equilibria formed on the fly, so no equilibrium or output array is held
 // (the D3Q27 kernel stays within 5 waves per SIMD); every output is the
 // same expression of the same operands as a per-population loop.
-template <class L, bool REF_PAIRS = false, bool FAST = false>
-__device__ __forceinline__ Macro collide_trt(float (&f)[L::Q], float tau_s, float tau_a, float gx, float gy,
-                                             float gz) {
-  const float omega_s = recip<FAST>(tau_s), omega_a = recip<FAST>(tau_a);
+template <class L, bool REF_PAIRS = false, bool FAST = false, bool FORCE = true>
+__device__ __forceinline__ Macro collide_trt_rate(float (&f)[L::Q], float omega_s, float omega_a, float gx, float gy,
+                                                  float gz) {
   const float pre_s = 1.0f - 0.5f * omega_s, pre_a = 1.0f - 0.5f * omega_a;
   float rho, jx, jy, jz, ux, uy, uz;
   density_momentum<L>(f, rho, jx, jy, jz);
-  guo_velocity<FAST>(rho, jx, jy, jz, gx, gy, gz, ux, uy, uz);
-  const float u_dot_g = ux * gx + uy * gy + uz * gz;
+  guo_velocity<FAST, FORCE>(rho, jx, jy, jz, gx, gy, gz, ux, uy, uz);
+  const float u_dot_g = FORCE ? ux * gx + uy * gy + uz * gz : 0.0f;
   const float usq = ux * ux + uy * uy + uz * uz;
   auto relax = [&](auto qc, float fq, float fo, float feq_q, float feo) {
     constexpr int q = decltype(qc)::value;
@@ -231,6 +243,7 @@ __device__ __forceinline__ Macro collide_trt(float (&f)[L::Q], float tau_s, floa
     const float f_asym = 0.5f * (fq - fo);
     const float fe_sym = 0.5f * (feq_q + feo);
     const float fe_asym = 0.5f * (feq_q - feo);
+    if constexpr (!FORCE) return fq - omega_s * (f_sym - fe_sym) - omega_a * (f_asym - fe_asym);
     const float cu = cdot<L, q>(ux, uy, uz);
     const float cg = cdot<L, q>(gx, gy, gz);
     const float F_asym = pre_a * L::w[q] * rho * (3.0f * cg);
@@ -250,14 +263,20 @@ __device__ __forceinline__ Macro collide_trt(float (&f)[L::Q], float tau_s, floa
   });
   return {rho, ux, uy, uz};
 }
+template <class L, bool REF_PAIRS = false, bool FAST = false>
+__device__ __forceinline__ Macro collide_trt(float (&f)[L::Q], float tau_s, float tau_a, float gx, float gy,
+                                             float gz) {
+  return collide_trt_rate<L, REF_PAIRS, FAST>(f, recip<FAST>(tau_s), recip<FAST>(tau_a), gx, gy, gz);
+}
 
 // D2Q9 MRT (Lallemand-Luo), in place (d2q9_collision_mrt.ispc:6-137).
 // With LES = true the shear rate comes from the Smagorinsky tau, the stress
 // taken from the moment deviations (sum c^2 (f - feq) = dm1 / 3,
 // Pi_xx - Pi_yy = dm7, Pi_xy = dm8) as in collide_mrt_d3q19.
-template <bool LES = false, bool FAST = false>
-__device__ __forceinline__ Macro collide_mrt_d2q9(float (&f)[9], float tau_shear, float tau_bulk, float gx,
-                                                  float gy, float cs = 0.0f) {
+// (s_nu = 1 / tau_shear, used with LES = false.)
+template <bool LES = false, bool FAST = false, bool FORCE = true>
+__device__ __forceinline__ Macro collide_mrt_d2q9_rate(float (&f)[9], float tau_shear, float s_nu, float tau_bulk,
+                                                       float gx, float gy, float cs) {
   const float s_e = 1.0f / tau_bulk, s_eps = 1.4f, s_q = 1.6f;
   const float f0 = f[0], f1 = f[1], f2 = f[2], f3 = f[3], f4 = f[4], f5 = f[5], f6 = f[6], f7 = f[7], f8 = f[8];
   float m0 = f0 + f1 + f2 + f3 + f4 + f5 + f6 + f7 + f8;
@@ -271,8 +290,8 @@ __device__ __forceinline__ Macro collide_mrt_d2q9(float (&f)[9], float tau_shear
   float m8 = (f5 - f6 + f7 - f8);
   const float rho = m0;
   const float inv_rho = recip<FAST>(rho);
-  const float ux = (m3 + 0.5f * rho * gx) * inv_rho;
-  const float uy = (m5 + 0.5f * rho * gy) * inv_rho;
+  const float ux = FORCE ? (m3 + 0.5f * rho * gx) * inv_rho : m3 * inv_rho;
+  const float uy = FORCE ? (m5 + 0.5f * rho * gy) * inv_rho : m5 * inv_rho;
   const float ux2 = ux * ux, uy2 = uy * uy, u2 = ux2 + uy2;
   const float meq1 = rho * (-2.0f + 3.0f * u2);
   const float meq2 = rho * (1.0f - 3.0f * u2);
@@ -292,22 +311,31 @@ __device__ __forceinline__ Macro collide_mrt_d2q9(float (&f)[9], float tau_shear
     const float disc = tau_shear * tau_shear + p_rho * q_stress;
     s_p = recip<FAST>(0.5f * (tau_shear + sqrt_of<FAST>(disc)));
   } else {
-    s_p = recip<FAST>(tau_shear);
+    s_p = s_nu;
   }
-  const float F_pre = 1.0f - 0.5f * s_p;
-  const float F_m3 = rho * gx, F_m5 = rho * gy;
-  const float F_m1 = 6.0f * (ux * F_m3 + uy * F_m5);
-  const float F_m2 = -6.0f * (ux * F_m3 + uy * F_m5);
-  const float F_m7 = 2.0f * (ux * F_m3 - uy * F_m5);
-  const float F_m8 = (ux * F_m5 + uy * F_m3);
-  m1 = m1 - s_e * (m1 - meq1) + F_pre * F_m1;
-  m2 = m2 - s_eps * (m2 - meq2) + F_pre * F_m2;
-  m3 = m3 + F_m3;
-  m4 = m4 - s_q * (m4 - meq4) + F_pre * (-F_m3);
-  m5 = m5 + F_m5;
-  m6 = m6 - s_q * (m6 - meq6) + F_pre * (-F_m5);
-  m7 = m7 - s_p * (m7 - meq7) + F_pre * F_m7;
-  m8 = m8 - s_p * (m8 - meq8) + F_pre * F_m8;
+  if constexpr (!FORCE) {
+    m1 = m1 - s_e * (m1 - meq1);
+    m2 = m2 - s_eps * (m2 - meq2);
+    m4 = m4 - s_q * (m4 - meq4);
+    m6 = m6 - s_q * (m6 - meq6);
+    m7 = m7 - s_p * (m7 - meq7);
+    m8 = m8 - s_p * (m8 - meq8);
+  } else {
+    const float F_pre = 1.0f - 0.5f * s_p;
+    const float F_m3 = rho * gx, F_m5 = rho * gy;
+    const float F_m1 = 6.0f * (ux * F_m3 + uy * F_m5);
+    const float F_m2 = -6.0f * (ux * F_m3 + uy * F_m5);
+    const float F_m7 = 2.0f * (ux * F_m3 - uy * F_m5);
+    const float F_m8 = (ux * F_m5 + uy * F_m3);
+    m1 = m1 - s_e * (m1 - meq1) + F_pre * F_m1;
+    m2 = m2 - s_eps * (m2 - meq2) + F_pre * F_m2;
+    m3 = m3 + F_m3;
+    m4 = m4 - s_q * (m4 - meq4) + F_pre * (-F_m3);
+    m5 = m5 + F_m5;
+    m6 = m6 - s_q * (m6 - meq6) + F_pre * (-F_m5);
+    m7 = m7 - s_p * (m7 - meq7) + F_pre * F_m7;
+    m8 = m8 - s_p * (m8 - meq8) + F_pre * F_m8;
+  }
   const float a9 = 1.0f / 9.0f, a18 = 1.0f / 18.0f, a36 = 1.0f / 36.0f, a6 = 1.0f / 6.0f, a12 = 1.0f / 12.0f;
   f[0] = a9 * m0 - a9 * m1 + a9 * m2;
   f[1] = a9 * m0 - a36 * m1 - a18 * m2 + a6 * m3 - a6 * m4 + 0.25f * m7;
@@ -319,6 +347,11 @@ __device__ __forceinline__ Macro collide_mrt_d2q9(float (&f)[9], float tau_shear
   f[7] = a9 * m0 + a18 * m1 + a36 * m2 - a6 * m3 - a12 * m4 - a6 * m5 - a12 * m6 + 0.25f * m8;
   f[8] = a9 * m0 + a18 * m1 + a36 * m2 + a6 * m3 + a12 * m4 - a6 * m5 - a12 * m6 - 0.25f * m8;
   return {rho, ux, uy, 0.0f};
+}
+template <bool LES = false, bool FAST = false>
+__device__ __forceinline__ Macro collide_mrt_d2q9(float (&f)[9], float tau_shear, float tau_bulk, float gx,
+                                                  float gy, float cs = 0.0f) {
+  return collide_mrt_d2q9_rate<LES, FAST>(f, tau_shear, LES ? 0.0f : recip<FAST>(tau_shear), tau_bulk, gx, gy, cs);
 }
 
 // A D3Q19 moment is "odd" when its basis polynomial changes sign under
@@ -874,6 +907,29 @@ __device__ __forceinline__ Macro collide_les(float (&f)[L::Q], float tau0, float
     guo_velocity<FAST>(rho, jx, jy, jz, gx, gy, gz, ux, uy, uz);
     return collide<L, COLL, false, FAST>(f, smagorinsky_tau_moments<L, FAST>(f, rho, ux, uy, uz, tau0, cs), gx, gy,
                                          gz);
+  }
+}
+
+// The D2Q9 collisions for kernels that take many steps: the rates of a
+// uniform tau are formed once (rate_s = 1 / tau, rate_a = 1 / trt_tau_a(tau))
+// and the force terms only where there is a force.
+template <int COLL, bool LES, bool FAST, bool FORCE>
+__device__ __forceinline__ Macro collide_d2q9_rates(float (&f)[9], float tau, float rate_s, float rate_a, float cs,
+                                                    float gx, float gy) {
+  using L = D2Q9;
+  if constexpr (COLL == kMRT) {
+    return collide_mrt_d2q9_rate<LES, FAST, FORCE>(f, tau, rate_s, kTauBulk2D, gx, gy, cs);
+  } else {
+    if constexpr (LES) {
+      float rho, jx, jy, jz, ux, uy, uz;
+      density_momentum<L>(f, rho, jx, jy, jz);
+      guo_velocity<FAST, FORCE>(rho, jx, jy, jz, gx, gy, 0.0f, ux, uy, uz);
+      const float te = smagorinsky_tau_moments<L, FAST>(f, rho, ux, uy, uz, tau, cs);
+      rate_s = recip<FAST>(te);
+      if constexpr (COLL == kTRT) rate_a = recip<FAST>(trt_tau_a(te));
+    }
+    if constexpr (COLL == kBGK) return collide_bgk_rate<L, FAST, FORCE>(f, rate_s, gx, gy, 0.0f);
+    else return collide_trt_rate<L, false, FAST, FORCE>(f, rate_s, rate_a, gx, gy, 0.0f);
   }
 }
 

@@ -389,9 +389,7 @@ __device__ __forceinline__ void gather(const StepArgs& a, const typename St::T* 
 // Multiply-adds are fused per source expression only ("contract on"): with
 // cross-statement fusion the inlet's fused pairs depended on the code around
 // the call, so kernels that differ only in addressing rounded it differently.
-template <class L>
-__device__ __forceinline__ void apply_inlet(const StepArgs& a, float (&f)[L::Q], int y, int n,
-                                            unsigned long long s_step) {
+__device__ __forceinline__ float inlet_velocity(const StepArgs& a, int y, int n, unsigned long long s_step) {
 #pragma clang fp contract(on)
   float ux = a.uin_x;
   if (a.inflow_parabolic) {
@@ -403,7 +401,13 @@ __device__ __forceinline__ void apply_inlet(const StepArgs& a, float (&f)[L::Q],
     const unsigned long long N = static_cast<unsigned long long>(a.nx) * a.ny * a.nz;
     ux = ux * (1.0f + a.turb_amp * rng_sym(a.turb_seed, s_step * N + static_cast<unsigned long long>(n)));
   }
-  const float uy = a.uin_y;
+  return ux;
+}
+
+// The inlet node's populations for the velocity (ux, uy, 0).
+template <class L>
+__device__ __forceinline__ void close_inlet(float (&f)[L::Q], float ux, float uy) {
+#pragma clang fp contract(on)
   if constexpr (L::Q == 9) {
     // d2q9_boundaries.ispc:43-81
     const float rho_in = (f[0] + f[2] + f[4] + 2.0f * (f[3] + f[6] + f[7])) / (1.0f - ux);
@@ -499,6 +503,12 @@ __device__ __forceinline__ void apply_inlet(const StepArgs& a, float (&f)[L::Q],
       }
     });
   }
+}
+
+template <class L>
+__device__ __forceinline__ void apply_inlet(const StepArgs& a, float (&f)[L::Q], int y, int n,
+                                            unsigned long long s_step) {
+  close_inlet<L>(f, inlet_velocity(a, y, n, s_step), a.uin_y);
 }
 
 // d2q9_boundaries.ispc:85-121 (pressure outlet, u_y = 0).
@@ -614,14 +624,15 @@ __device__ __forceinline__ void form_s(const StepArgs& a, const typename St::T* 
 // called per link with the midpoint offset from the centre.  The midpoint
 // test rounds as the host's link builder (no fused multiply-add).  n is the
 // node's index: with the bounce masks built, the walls come from its mask
-// (bit opp(q) of an in-range neighbour), not from reading the neighbours'
-// cell types.  Only for kClsSlow nodes (other nodes have no wall neighbour).
+// (bit opp(q) of an in-range neighbour; known_bm where the caller holds it),
+// not from reading the neighbours' cell types.  Only for kClsSlow nodes (other nodes have no wall neighbour).
 template <class L, class OnLink>
 __device__ __forceinline__ void for_each_mem_link(const StepArgs& a, int x, int y, int z, int n, float ccx,
-                                                  float ccy, float ccz, float r_max, OnLink&& on_link) {
+                                                  float ccy, float ccz, float r_max, OnLink&& on_link,
+                                                  const uint32_t* known_bm = nullptr) {
   const float r_max_sq = r_max * r_max;
-  const bool use_bm = a.bmask != nullptr;
-  const uint32_t bm = use_bm ? a.bmask[n] : 0u;
+  const bool use_bm = known_bm || a.bmask != nullptr;
+  const uint32_t bm = known_bm ? *known_bm : (use_bm ? a.bmask[n] : 0u);
   static_for<L::Q>([&](auto qc) {
     constexpr int q = decltype(qc)::value;
     if constexpr (q > 0) {
@@ -662,7 +673,7 @@ __device__ __forceinline__ bool is_fluid(const StepArgs& a, int n) {
 template <class L>
 __device__ __forceinline__ void mem_node(const StepArgs& a, int x, int y, int z, int n, const float (&f)[L::Q],
                                          float ccx, float ccy, float ccz, float r_max, double& s0, double& s1,
-                                         double& s2) {
+                                         double& s2, const uint32_t* known_bm = nullptr) {
   for_each_mem_link<L>(a, x, y, z, n, ccx, ccy, ccz, r_max, [&](auto qc, float rx, float ry) {
     constexpr int q = decltype(qc)::value;
     constexpr int cx = L::cx[q], cy = L::cy[q], cz = L::cz[q];
@@ -672,7 +683,7 @@ __device__ __forceinline__ void mem_node(const StepArgs& a, int x, int y, int z,
     s1 += dfy;
     if constexpr (L::D == 2) s2 += static_cast<double>(rx * dfy - ry * dfx);
     else s2 += static_cast<double>(2.0f * f[q] * static_cast<float>(cz));
-  });
+  }, known_bm);
 }
 
 // Sum over the 64 lanes of a wave in a fixed butterfly order; lane 0's
@@ -870,91 +881,6 @@ __global__ __launch_bounds__(256) WAKE_STEP_ATTR void k_step(const StepArgs a, c
         St::template st<L, q>(aout, q * S + n, f[q]);
       });
     }
-  }
-}
-
-// ------------------------------------------- fully periodic D2Q9, T steps
-// A fully periodic D2Q9 domain without solid, inlet or outlet nodes (every
-// class byte zero) streams by a plain periodic shift, so kTbSteps steps can
-// run in one launch: each work-group loads a (16 + 2 T)^2 tile of A_{k-1}
-// around its 16 x 16 nodes into LDS, pull-collides T times in LDS (the
-// valid region shrinks by one node per step), and stores A_{k-1+T} of its
-// 16 x 16 nodes.  One thread per tile node (1,024 threads, 16 waves), so
-// each SIMD holds four of the work-group's waves to overlap LDS latency.  Every node update is the same pull, collision and storage
-// rounding as one k_step launch, so the result is the same as T launches;
-// the launch cost and the HBM traffic are paid once per T steps.
-inline constexpr int kTbTile = 16;
-
-template <class St, class L, int q>
-__device__ __forceinline__ float tb_get(typename St::T v) {
-  if constexpr (sizeof(typename St::T) == 4) {
-    return v;
-  } else {
-    return St::template from_dev_bits<L, q>(__builtin_bit_cast(unsigned short, v));
-  }
-}
-template <class St, class L, int q>
-__device__ __forceinline__ typename St::T tb_put(float v) {
-  if constexpr (sizeof(typename St::T) == 4) {
-    return v;
-  } else {
-    return __builtin_bit_cast(typename St::T, St::template dev_bits<L, q>(v));
-  }
-}
-
-inline constexpr int kTbWidth = kTbTile + 2 * kTbSteps;  // 32
-inline constexpr int kTbThreads = kTbWidth * kTbWidth;     // one per tile node
-
-template <class St, int COLL, bool LES>
-__global__ __launch_bounds__(kTbThreads) void k_step_tb2d(const StepArgs a, const typename St::T* __restrict__ ain,
-                                                          typename St::T* __restrict__ aout) {
-  using L = D2Q9;
-  using T = typename St::T;
-  constexpr int W = kTbWidth;
-  static_assert((W & (W - 1)) == 0, "tile width");
-  __shared__ T tile[2][L::Q][W * W];
-  const int x0 = blockIdx.x * kTbTile - kTbSteps, y0 = blockIdx.y * kTbTile - kTbSteps;
-  const long long S = a.stride;
-  const int c = threadIdx.x;  // this thread's tile node
-  const int i = c & (W - 1), j = c / W;
-  {
-    const int gx = ((x0 + i) % a.nx + a.nx) % a.nx;
-    const int gy = ((y0 + j) % a.ny + a.ny) % a.ny;
-    const long long n = static_cast<long long>(gy) * a.nx + gx;
-    static_for<L::Q>([&](auto qc) {
-      constexpr int q = decltype(qc)::value;
-      tile[0][q][c] = ain[q * S + n];
-    });
-  }
-  __syncthreads();
-#pragma unroll 1
-  for (int s = 1; s <= kTbSteps; ++s) {
-    const int src = (s - 1) & 1, dst = s & 1;
-    if (i >= s && i < W - s && j >= s && j < W - s) {
-      float f[L::Q];
-      static_for<L::Q>([&](auto qc) {
-        constexpr int q = decltype(qc)::value;
-        f[q] = tb_get<St, L, q>(tile[src][q][(j - L::cy[q]) * W + (i - L::cx[q])]);
-      });
-      Macro m;
-      if constexpr (LES) m = collide_les<L, COLL, St::kFast>(f, a.tau, a.cs, a.gx, a.gy, a.gz);
-      else m = collide<L, COLL, false, St::kFast>(f, a.tau, a.gx, a.gy, a.gz);
-      flag_nonfinite(a, m.rho);
-      static_for<L::Q>([&](auto qc) {
-        constexpr int q = decltype(qc)::value;
-        tile[dst][q][c] = tb_put<St, L, q>(f[q]);
-      });
-    }
-    __syncthreads();
-  }
-  const int li = i - kTbSteps, lj = j - kTbSteps;
-  const int gx = blockIdx.x * kTbTile + li, gy = blockIdx.y * kTbTile + lj;
-  if (li >= 0 && li < kTbTile && lj >= 0 && lj < kTbTile && gx < a.nx && gy < a.ny) {
-    const long long n = static_cast<long long>(gy) * a.nx + gx;
-    static_for<L::Q>([&](auto qc) {
-      constexpr int q = decltype(qc)::value;
-      aout[q * S + n] = tile[kTbSteps & 1][q][c];
-    });
   }
 }
 

@@ -71,9 +71,11 @@ __device__ __forceinline__ float thermal_t(const float (&g)[D2Q5::Q]) {
   return T;
 }
 
-// Collide a fluid node's f (per-node Boussinesq force) and g.
+// Collide a fluid node's f (per-node Boussinesq force) and g; rate_s, rate_a
+// as in collide_d2q9_rates, omega_g = 1 / tau_g.
 template <int COLL>
-__device__ __forceinline__ void thermal_collide(const StepArgs& a, float (&f)[D2Q9::Q], float (&g)[D2Q5::Q]) {
+__device__ __forceinline__ void thermal_collide_rates(const StepArgs& a, float rate_s, float rate_a, float omega_g,
+                                                      float (&f)[D2Q9::Q], float (&g)[D2Q5::Q]) {
   const float T = thermal_t(g);
   const float gyn = a.gy + a.gbeta * (T - a.t_ref);
   float rho = 0.0f, jx = 0.0f, jy = 0.0f;
@@ -87,14 +89,17 @@ __device__ __forceinline__ void thermal_collide(const StepArgs& a, float (&f)[D2
   const float inv_rho = 1.0f / rho;
   const float ux = (jx + 0.5f * rho * a.gx) * inv_rho;
   const float uy = (jy + 0.5f * rho * gyn) * inv_rho;
-  collide<D2Q9, COLL>(f, a.tau, a.gx, gyn, 0.0f);
-  const float omega_g = 1.0f / a.tau_g;
+  collide_d2q9_rates<COLL, false, false, true>(f, a.tau, rate_s, rate_a, 0.0f, a.gx, gyn);
   static_for<D2Q5::Q>([&](auto qc) {
     constexpr int q = decltype(qc)::value;
     const float cu = static_cast<float>(D2Q5::cx[q]) * ux + static_cast<float>(D2Q5::cy[q]) * uy;
     const float geq = D2Q5::w[q] * T * (1.0f + 3.0f * cu);
     g[q] = g[q] - omega_g * (g[q] - geq);
   });
+}
+template <int COLL>
+__device__ __forceinline__ void thermal_collide(const StepArgs& a, float (&f)[D2Q9::Q], float (&g)[D2Q5::Q]) {
+  thermal_collide_rates<COLL>(a, 1.0f / a.tau, COLL == kTRT ? 1.0f / trt_tau_a(a.tau) : 0.0f, 1.0f / a.tau_g, f, g);
 }
 
 // One node of the coupled step: S of f and g (pulled from A, or read from a

@@ -159,11 +159,10 @@ class _Domain:
         self._c(self._L.wake_domain_set_block_x(self._h, bx), "set_block_x")
 
     def set_multistep(self, on=True):
-        """Let run() take 8 steps per launch where the domain allows it
-        (fully periodic 2D, all cells Fluid, no open boundary, force probe
-        or temperature) and single launches are bound by the launch rate
-        (up to 2^21 nodes in FP32, 2^17 with 16-bit storage); the result is
-        the same as single steps."""
+        """Let run() take up to 8 steps per launch (2D domains without curved
+        links and without the convective outlet, and not timed runs; 16-bit
+        storage up to 2^23 nodes, 2^19 with temperature, BF16 temperature
+        not); the result is the same as single steps."""
         self._c(self._L.wake_domain_set_multistep(self._h, int(bool(on))), "set_multistep")
 
     # --------------------------------------------------------------- steps
