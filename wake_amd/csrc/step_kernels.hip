@@ -48,20 +48,36 @@ __global__ __launch_bounds__(256) void k_diag_partial(const uint8_t* __restrict_
   }
 }
 
-__global__ void k_diag_final(const double* __restrict__ partial, int nblocks, double* __restrict__ out) {
-  if (threadIdx.x != 0 || blockIdx.x != 0) return;
+// The partials in one work-group, each lane's in block order, then the tree:
+// 5 us for 1024 blocks, where one lane walking them took 113 us (a chain of
+// dependent memory round trips).
+__global__ __launch_bounds__(256) void k_diag_final(const double* __restrict__ partial, int nblocks,
+                                                    double* __restrict__ out) {
+  __shared__ double sm[256], se[256], sx[256];
   double m = 0.0, e = 0.0, mx = 0.0;
-  for (int b = 0; b < nblocks; ++b) {
+  for (int b = threadIdx.x; b < nblocks; b += 256) {
     m += partial[3 * b];
     e += partial[3 * b + 1];
     mx = fmax(mx, partial[3 * b + 2]);
   }
-  out[0] = m;
-  out[1] = e;
-  out[2] = mx;
+  sm[threadIdx.x] = m;
+  se[threadIdx.x] = e;
+  sx[threadIdx.x] = mx;
+  __syncthreads();
+  for (int w = 128; w > 0; w >>= 1) {
+    if (threadIdx.x < w) {
+      sm[threadIdx.x] += sm[threadIdx.x + w];
+      se[threadIdx.x] += se[threadIdx.x + w];
+      sx[threadIdx.x] = fmax(sx[threadIdx.x], sx[threadIdx.x + w]);
+    }
+    __syncthreads();
+  }
+  if (threadIdx.x == 0) {
+    out[0] = sm[0];
+    out[1] = se[0];
+    out[2] = sx[0];
+  }
 }
-
-
 
 hipError_t launch_build_class(int lattice, const StepArgs& a, uint8_t* cls, uint32_t* bmask, hipStream_t s) {
   switch (lattice) {
@@ -197,7 +213,7 @@ hipError_t launch_count_nonfinite(const float* rho, const float* speed, long lon
 hipError_t launch_diagnostics(const uint8_t* flags, const float* rho, const float* speed, long long n,
                               double* partial, int nblocks, double* out3, hipStream_t s) {
   k_diag_partial<<<nblocks, 256, 0, s>>>(flags, rho, speed, n, partial);
-  k_diag_final<<<1, 64, 0, s>>>(partial, nblocks, out3);
+  k_diag_final<<<1, 256, 0, s>>>(partial, nblocks, out3);
   return hipGetLastError();
 }
 
