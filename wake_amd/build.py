@@ -43,11 +43,13 @@ HOST_FLAGS = ["-O2", "-std=c++20", "-fPIC", "-ffp-contract=off", f"--offload-arc
 SOURCES = [
     "step_d3q19.hip", "step_d3q27.hip", "step_d2q9.hip", "tile2d.hip", "step_kernels.hip", "thermal.hip", "analytics.hip",
     "ispc_compat.hip", "batch.hip", "domain.cpp", "capi.cpp", "lattice_grid.cpp", "runner.cpp", "batch_host.cpp",
-    "host_api.cpp", "geometry.hip", "export.cpp", "thermal_solver.cpp", "hbm_probe.hip",
+    "host_api.cpp", "host_pipe.cpp", "geometry.hip", "state_init.hip", "export.cpp", "thermal_solver.cpp", "hbm_probe.hip",
 ]
-# The voxelizer's overlap test and the link builder's wall fractions must
-# round every product and sum on its own, with IEEE division and sqrt.
-EXTRA_FLAGS = {"geometry.hip": ["-ffp-contract=off", "-fhip-fp32-correctly-rounded-divide-sqrt"]}
+# The voxelizer's overlap test, the link builder's wall fractions and the
+# initial equilibria must round every product and sum on its own, with IEEE
+# division and sqrt.
+EXACT_FLAGS = ["-ffp-contract=off", "-fhip-fp32-correctly-rounded-divide-sqrt"]
+EXTRA_FLAGS = {"geometry.hip": EXACT_FLAGS, "state_init.hip": EXACT_FLAGS}
 
 
 def _headers_mtime():

@@ -208,25 +208,21 @@ int wake_domain_synchronize(wake_domain* d) {
 }
 int wake_domain_read(wake_domain* d, int field, float* out) {
   return guard(d, [&](wake_hip::Domain& g) {
-    const size_t N = g.total_nodes();
-    const float* src = nullptr;
-    size_t n = N;
     switch (field) {
-      case WAKE_FIELD_RHO: src = g.rho(); break;
-      case WAKE_FIELD_UX: src = g.ux(); break;
-      case WAKE_FIELD_UY: src = g.uy(); break;
-      case WAKE_FIELD_UZ: src = g.uz(); break;
-      case WAKE_FIELD_SPEED: src = g.speed(); break;
-      case WAKE_FIELD_F_SRC: src = g.f_src(); n = N * g.lattice(); break;
-      case WAKE_FIELD_F_DST: src = g.f_dst(); n = N * g.lattice(); break;
-      case WAKE_FIELD_TEMPERATURE: src = g.temperature(); break;
-      case WAKE_FIELD_OMEGA_X: src = g.analytics(0); break;
-      case WAKE_FIELD_OMEGA_Y: src = g.analytics(1); break;
-      case WAKE_FIELD_OMEGA_Z: src = g.analytics(2); break;
-      case WAKE_FIELD_Q_CRITERION: src = g.analytics(3); break;
+      case WAKE_FIELD_RHO: g.read_field(0, out); break;
+      case WAKE_FIELD_UX: g.read_field(1, out); break;
+      case WAKE_FIELD_UY: g.read_field(2, out); break;
+      case WAKE_FIELD_UZ: g.read_field(3, out); break;
+      case WAKE_FIELD_SPEED: g.read_field(4, out); break;
+      case WAKE_FIELD_F_SRC: g.read_f_src(out); break;
+      case WAKE_FIELD_F_DST: g.read_f_dst(out); break;
+      case WAKE_FIELD_TEMPERATURE: g.read_field(5, out); break;
+      case WAKE_FIELD_OMEGA_X: g.read_analytics(0, out); break;
+      case WAKE_FIELD_OMEGA_Y: g.read_analytics(1, out); break;
+      case WAKE_FIELD_OMEGA_Z: g.read_analytics(2, out); break;
+      case WAKE_FIELD_Q_CRITERION: g.read_analytics(3, out); break;
       default: throw wake_hip::HipError("unknown field");
     }
-    std::memcpy(out, src, n * sizeof(float));
   });
 }
 int wake_domain_read_cell_types(wake_domain* d, uint8_t* out) {

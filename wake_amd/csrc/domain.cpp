@@ -1,5 +1,6 @@
 // domain.cpp -- host side of a device-resident lattice domain.
 #include "domain.hpp"
+#include "host_pipe.hpp"
 
 #include <algorithm>
 #include <cmath>
@@ -131,21 +132,19 @@ void Domain::allocate_and_initialize() {
   d_nonfinite_ = static_cast<int*>(alloc(sizeof(int)));
   d_nfcount_ = static_cast<unsigned long long*>(alloc(2 * sizeof(unsigned long long)));
   flags_.assign(N_, kFluid);
-  h_rho_.resize(N_);
-  h_ux_.resize(N_);
-  h_uy_.resize(N_);
-  h_uz_.resize(N_);
-  h_speed_.resize(N_);
   initialize(1.0f, 0.0f, 0.0f, 0.0f);
 }
 
 Domain::~Domain() { release(); }
 
 void Domain::release() noexcept {
+  bool last = false;
   {
     std::lock_guard<std::mutex> lock(g_live_mutex);
     g_live.erase(std::remove(g_live.begin(), g_live.end(), this), g_live.end());
+    last = g_live.empty();
   }
+  if (last) trim_host_pipe();
   if (stream_) (void)hipStreamSynchronize(stream_);
   for (hipEvent_t e : kev_) (void)hipEventDestroy(e);
   kev_.clear();
@@ -220,11 +219,6 @@ void Domain::initialize(float rho, float ux, float uy, float uz) {
   flags_dirty_ = cls_dirty_ = true;
   ++flags_version_;
   const float sp = std::sqrt(u_sq);
-  std::fill(h_rho_.begin(), h_rho_.end(), rho);
-  std::fill(h_ux_.begin(), h_ux_.end(), ux);
-  std::fill(h_uy_.begin(), h_uy_.end(), uy);
-  std::fill(h_uz_.begin(), h_uz_.end(), uz);
-  std::fill(h_speed_.begin(), h_speed_.end(), sp);
   const float vals[5] = {rho, ux, uy, uz, sp};
   float* dst[5] = {d_rho_, d_ux_, d_uy_, d_uz_, d_speed_};
   for (int k = 0; k < 5; ++k) {
@@ -232,7 +226,8 @@ void Domain::initialize(float rho, float ux, float uy, float uz) {
     std::memcpy(&b, &vals[k], 4);
     check(hipMemsetD32Async(static_cast<hipDeviceptr_t>(dst[k]), b, N_, stream_), "fill");
   }
-  fields_valid_ = true;
+  dfields_valid_ = true;
+  mirrors_ = 0;
   fsrc_valid_ = fdst_valid_ = false;
   sout_is_fsrc_ = false;
   clear_nonfinite();
@@ -240,90 +235,61 @@ void Domain::initialize(float rho, float ux, float uy, float uz) {
   if (probe_) probe_restart();
 }
 
-void Domain::upload_state_from_host(const std::vector<float>& f_ref) {
+// The state now is a materialised S in buffer 0, formed on the device.
+void Domain::state_set() {
   ++version_;
-  // f_ref: Q planes of N (reference layout) -> storage format, padded stride.
-  const LatTab L = tab(lattice_);
-  std::vector<char> host(static_cast<size_t>(Q_) * stride_ * elem_, 0);
-  for (int q = 0; q < Q_; ++q) {
-    const float* src = f_ref.data() + static_cast<size_t>(q) * N_;
-    char* dst = host.data() + static_cast<size_t>(q) * stride_ * elem_;
-    if (storage_ == kStoreF32) {
-      std::memcpy(dst, src, N_ * 4);
-    } else {
-      uint16_t* d16 = reinterpret_cast<uint16_t*>(dst);
-      for (size_t i = 0; i < N_; ++i)
-        d16[i] = storage_ == kStoreF16 ? to_half_bits(src[i] - L.w[q]) : to_bf16_bits(src[i] - L.w[q]);
-    }
-  }
-  check(hipMemcpyAsync(buf_[0], host.data(), host.size(), hipMemcpyHostToDevice, stream_), "upload");
   clear_nonfinite();
-  // convective outlet store = S_0 on the x = nx - 1 plane
-  upload_prev([&](size_t row, int q) { return f_ref[static_cast<size_t>(q) * N_ + row * nx_ + (nx_ - 1)]; });
-  check(hipStreamSynchronize(stream_), "upload");
   s_buf_ = 0;
   a_buf_ = -1;
-  h_fsrc_ = f_ref;
-  fsrc_valid_ = (storage_ == kStoreF32);
-  sout_is_fsrc_ = false;
-  fdst_valid_ = false;
+  fsrc_valid_ = fdst_valid_ = sout_is_fsrc_ = false;
   if (probe_) probe_restart();  // the state the samples were taken of is gone
+}
+
+float* Domain::planes_scratch() {
+  if (!d_sout_) d_sout_ = static_cast<float*>(alloc(static_cast<size_t>(Q_) * N_ * sizeof(float)));
+  return d_sout_;
 }
 
 // lattice_grid_3d.cpp:95-131 with the per-node values as arrays; cell types
 // are left untouched.
 void Domain::initialize_fields(const float* rho, const float* ux, const float* uy, const float* uz) {
-  const LatTab L = tab(lattice_);
   step_count_ = 0;
-  std::vector<float> f(static_cast<size_t>(Q_) * N_);
-  for (size_t i = 0; i < N_; ++i) {
-    const float r = rho[i], a = ux[i], b = uy[i], c = (dim_ == 2 || !uz) ? 0.0f : uz[i];
-    const float u_sq = dim_ == 2 ? a * a + b * b : a * a + b * b + c * c;
-    h_rho_[i] = r;
-    h_ux_[i] = a;
-    h_uy_[i] = b;
-    h_uz_[i] = c;
-    h_speed_[i] = std::sqrt(u_sq);
-    for (int q = 0; q < Q_; ++q) {
-      const float ci_u = dim_ == 2 ? static_cast<float>(L.cx[q]) * a + static_cast<float>(L.cy[q]) * b
-                                   : static_cast<float>(L.cx[q]) * a + static_cast<float>(L.cy[q]) * b +
-                                         static_cast<float>(L.cz[q]) * c;
-      f[static_cast<size_t>(q) * N_ + i] = L.w[q] * r * (1.0f + 3.0f * ci_u + 4.5f * ci_u * ci_u - 1.5f * u_sq);
-    }
+  float* dst[4] = {d_rho_, d_ux_, d_uy_, d_uz_};
+  const float* src[4] = {rho, ux, uy, dim_ == 2 ? nullptr : uz};
+  for (int k = 0; k < 4; ++k) {
+    if (src[k]) check(hipMemcpyAsync(dst[k], src[k], N_ * sizeof(float), hipMemcpyHostToDevice, stream_), "upload");
+    else check(hipMemsetAsync(dst[k], 0, N_ * sizeof(float), stream_), "upload");
   }
-  upload_state_from_host(f);
-  float* dst[5] = {d_rho_, d_ux_, d_uy_, d_uz_, d_speed_};
-  const std::vector<float>* src[5] = {&h_rho_, &h_ux_, &h_uy_, &h_uz_, &h_speed_};
-  for (int k = 0; k < 5; ++k)
-    check(hipMemcpyAsync(dst[k], src[k]->data(), N_ * 4, hipMemcpyHostToDevice, stream_), "upload");
-  check(hipStreamSynchronize(stream_), "upload");
-  fields_valid_ = true;
+  check(launch_init_fields(lattice_, storage_, d_rho_, d_ux_, d_uy_, d_uz_, d_speed_, buf_[0], stride_, d_prev_, nx_,
+                           static_cast<int>(N_), stream_),
+        "initialize");
+  state_set();
+  check(hipStreamSynchronize(stream_), "upload");  // the caller's arrays are free again
+  mirrors_ = 0;
+  dfields_valid_ = true;  // the fields given, not the moments of their equilibria
 }
 
 void Domain::set_populations(const float* f_ref) {
   before_config_change();
-  std::vector<float> f(f_ref, f_ref + static_cast<size_t>(Q_) * N_);
-  upload_state_from_host(f);
+  check(hipMemcpyAsync(planes_scratch(), f_ref, static_cast<size_t>(Q_) * N_ * sizeof(float), hipMemcpyHostToDevice,
+                       stream_),
+        "upload");
+  check(launch_init_planes(lattice_, storage_, d_sout_, 0.0f, 0, buf_[0], stride_, d_prev_, nx_, static_cast<int>(N_),
+                           stream_),
+        "set populations");
+  state_set();
+  check(hipStreamSynchronize(stream_), "upload");
   invalidate_mirrors();
-  fsrc_valid_ = (storage_ == kStoreF32);
 }
 
 // Seeded uniform noise U(-a, a) on every population, counter = node * Q + q.
 void Domain::add_noise(float amplitude, uint64_t seed) {
-  std::vector<float> f(f_src(), f_src() + static_cast<size_t>(Q_) * N_);
-  for (size_t i = 0; i < N_; ++i)
-    for (int q = 0; q < Q_; ++q) {
-      const uint64_t h = splitmix64(seed ^ (static_cast<uint64_t>(i) * Q_ + q));
-      const double u = static_cast<double>(h >> 40) * (1.0 / 16777216.0);
-      f[static_cast<size_t>(q) * N_ + i] += amplitude * static_cast<float>(2.0 * u - 1.0);
-    }
-  const uint64_t keep = step_count_;
-  const bool fv = fields_valid_, dfv = dfields_valid_;
-  upload_state_from_host(f);
-  step_count_ = keep;
-  if (probe_) probe_restart();
-  fields_valid_ = fv;
-  dfields_valid_ = dfv;
+  form_planes();
+  check(launch_init_planes(lattice_, storage_, d_sout_, amplitude, seed, buf_[0], stride_, d_prev_, nx_,
+                           static_cast<int>(N_), stream_),
+        "noise");
+  state_set();
+  check(hipStreamSynchronize(stream_), "noise");
 }
 
 // ------------------------------------------------------------- cell types
@@ -921,7 +887,7 @@ void Domain::synchronize() { check(hipStreamSynchronize(stream_), "synchronize")
 
 // ------------------------------------------------------------- read-back
 void Domain::ensure_device_fields() {
-  if (fields_valid_ || dfields_valid_) return;
+  if (dfields_valid_) return;
   sync_device_config();
   StepArgs a = args(false);
   a.rho = d_rho_;
@@ -940,50 +906,74 @@ void Domain::ensure_device_fields() {
   dfields_valid_ = true;
 }
 
-void Domain::ensure_fields() {
-  if (fields_valid_) return;
+float* Domain::device_array(int which) {
+  float* d[6] = {d_rho_, d_ux_, d_uy_, d_uz_, d_speed_, d_temp_};
+  return d[which];
+}
+
+const float* Domain::mirror(int which) {
+  if (!(mirrors_ & (1u << which))) {
+    ensure_device_fields();
+    h_field_[which].resize(N_);
+    device_to_host(h_field_[which].data(), device_array(which), N_ * sizeof(float), stream_);
+    mirrors_ |= 1u << which;
+  }
+  return h_field_[which].data();
+}
+
+void Domain::read_field(int which, float* out) {
+  if (which == 5 && !thermal_) throw HipError("temperature is not enabled on this domain");
+  if (mirrors_ & (1u << which)) {
+    std::memcpy(out, h_field_[which].data(), N_ * sizeof(float));
+    return;
+  }
   ensure_device_fields();
-  if (thermal_) check(hipMemcpyAsync(h_temp_.data(), d_temp_, N_ * 4, hipMemcpyDeviceToHost, stream_), "d2h");
-  float* d[5] = {d_rho_, d_ux_, d_uy_, d_uz_, d_speed_};
-  std::vector<float>* h[5] = {&h_rho_, &h_ux_, &h_uy_, &h_uz_, &h_speed_};
-  for (int k = 0; k < 5; ++k) check(hipMemcpyAsync(h[k]->data(), d[k], N_ * 4, hipMemcpyDeviceToHost, stream_), "d2h");
-  check(hipStreamSynchronize(stream_), "readback");
-  fields_valid_ = true;
+  device_to_host(out, device_array(which), N_ * sizeof(float), stream_);
 }
 
 // lattice_grid_3d.cpp:292-299: unforced moments of f_src, then |u|.
 void Domain::update_macroscopic() {
   const float keep[3] = {g_last_[0], g_last_[1], g_last_[2]};
   g_last_[0] = g_last_[1] = g_last_[2] = 0.0f;
-  fields_valid_ = dfields_valid_ = false;
-  ensure_fields();
+  dfields_valid_ = false;
+  mirrors_ = 0;
+  ensure_device_fields();
   g_last_[0] = keep[0];
   g_last_[1] = keep[1];
   g_last_[2] = keep[2];
 }
 
-const float* Domain::analytics(int which) {
+void Domain::ensure_analytics(int which) {
   if (which < 0 || which > 3) throw HipError("unknown analytics field");
   if (dim_ == 2 && which != 2) throw HipError("a 2D domain has only the z vorticity");
-  if (!an_valid_) {
-    ensure_fields();
-    const int k0 = dim_ == 2 ? 2 : 0, k1 = dim_ == 2 ? 2 : 3;
-    for (int k = k0; k <= k1; ++k)
-      if (!d_an_[k]) {
-        d_an_[k] = static_cast<float*>(alloc(N_ * sizeof(float)));
-        h_an_[k].resize(N_);
-      }
-    if (dim_ == 2)
-      check(launch_vorticity_2d(d_ux_, d_uy_, d_an_[2], nx_, ny_, stream_), "vorticity");
-    else
-      check(launch_vorticity_q_3d(d_ux_, d_uy_, d_uz_, d_an_[0], d_an_[1], d_an_[2], d_an_[3], nx_, ny_, nz_, stream_),
-            "vorticity");
-    for (int k = k0; k <= k1; ++k)
-      check(hipMemcpyAsync(h_an_[k].data(), d_an_[k], N_ * sizeof(float), hipMemcpyDeviceToHost, stream_), "d2h");
-    check(hipStreamSynchronize(stream_), "vorticity");
-    an_valid_ = true;
+  if (an_valid_) return;
+  ensure_device_fields();
+  const int k0 = dim_ == 2 ? 2 : 0, k1 = dim_ == 2 ? 2 : 3;
+  for (int k = k0; k <= k1; ++k)
+    if (!d_an_[k]) d_an_[k] = static_cast<float*>(alloc(N_ * sizeof(float)));
+  if (dim_ == 2)
+    check(launch_vorticity_2d(d_ux_, d_uy_, d_an_[2], nx_, ny_, stream_), "vorticity");
+  else
+    check(launch_vorticity_q_3d(d_ux_, d_uy_, d_uz_, d_an_[0], d_an_[1], d_an_[2], d_an_[3], nx_, ny_, nz_, stream_),
+          "vorticity");
+  an_valid_ = true;
+  an_mirrors_ = 0;
+}
+
+const float* Domain::analytics(int which) {
+  ensure_analytics(which);
+  if (!(an_mirrors_ & (1u << which))) {
+    h_an_[which].resize(N_);
+    device_to_host(h_an_[which].data(), d_an_[which], N_ * sizeof(float), stream_);
+    an_mirrors_ |= 1u << which;
   }
   return h_an_[which].data();
+}
+
+void Domain::read_analytics(int which, float* out) {
+  ensure_analytics(which);
+  if (an_mirrors_ & (1u << which)) std::memcpy(out, h_an_[which].data(), N_ * sizeof(float));
+  else device_to_host(out, d_an_[which], N_ * sizeof(float), stream_);
 }
 
 const float* Domain::device_field(int which) {
@@ -998,65 +988,75 @@ const uint8_t* Domain::device_cell_types() {
   return d_flags_;
 }
 
-const float* Domain::rho() { ensure_fields(); return h_rho_.data(); }
-const float* Domain::ux() { ensure_fields(); return h_ux_.data(); }
-const float* Domain::uy() { ensure_fields(); return h_uy_.data(); }
-const float* Domain::uz() { ensure_fields(); return h_uz_.data(); }
-const float* Domain::speed() { ensure_fields(); return h_speed_.data(); }
+const float* Domain::rho() { return mirror(0); }
+const float* Domain::ux() { return mirror(1); }
+const float* Domain::uy() { return mirror(2); }
+const float* Domain::uz() { return mirror(3); }
+const float* Domain::speed() { return mirror(4); }
+
+// S_k in the reference layout (FP32 planes of N) in d_sout_.
+void Domain::form_planes() {
+  sync_device_config();
+  StepArgs a = args(false);
+  a.s_out = planes_scratch();
+  const bool from_s = s_buf_ >= 0;
+  check(launch_readback(lattice_, storage_, from_s, a, buf_[from_s ? s_buf_ : a_buf_], stream_), "readback");
+  sout_is_fsrc_ = false;
+}
 
 const float* Domain::f_src() {
   if (fsrc_valid_) return h_fsrc_.data();
-  sync_device_config();
-  if (!d_sout_) d_sout_ = static_cast<float*>(alloc(static_cast<size_t>(Q_) * N_ * 4));
-  StepArgs a = args(false);
-  a.rho = d_rho_;
-  a.ux = d_ux_;
-  a.uy = d_uy_;
-  a.uz = d_uz_;
-  a.speed = d_speed_;
-  a.s_out = d_sout_;
-  const bool from_s = s_buf_ >= 0;
-  check(launch_readback(lattice_, storage_, from_s, a, buf_[from_s ? s_buf_ : a_buf_], stream_), "readback");
+  form_planes();
   h_fsrc_.resize(static_cast<size_t>(Q_) * N_);
-  check(hipMemcpyAsync(h_fsrc_.data(), d_sout_, h_fsrc_.size() * 4, hipMemcpyDeviceToHost, stream_), "d2h");
-  if (!fields_valid_) {
-    float* d[5] = {d_rho_, d_ux_, d_uy_, d_uz_, d_speed_};
-    std::vector<float>* h[5] = {&h_rho_, &h_ux_, &h_uy_, &h_uz_, &h_speed_};
-    for (int k = 0; k < 5; ++k)
-      check(hipMemcpyAsync(h[k]->data(), d[k], N_ * 4, hipMemcpyDeviceToHost, stream_), "d2h");
-    fields_valid_ = true;
-  }
-  check(hipStreamSynchronize(stream_), "readback");
+  device_to_host(h_fsrc_.data(), d_sout_, h_fsrc_.size() * sizeof(float), stream_);
   fsrc_valid_ = true;
   sout_is_fsrc_ = true;
   return h_fsrc_.data();
 }
 
+void Domain::read_f_src(float* out) {
+  const size_t bytes = static_cast<size_t>(Q_) * N_ * sizeof(float);
+  if (fsrc_valid_) {
+    std::memcpy(out, h_fsrc_.data(), bytes);
+    return;
+  }
+  form_planes();
+  device_to_host(out, d_sout_, bytes, stream_);
+}
+
 // After step k the reference's f_dst holds A_{k-1}; before any step it holds
 // the initial state.
-const float* Domain::f_dst() {
-  if (fdst_valid_) return h_fdst_.data();
-  if (a_buf_ < 0) {
-    h_fdst_.assign(f_src(), f_src() + static_cast<size_t>(Q_) * N_);
-    fdst_valid_ = true;
-    return h_fdst_.data();
-  }
-  if (!d_sout_) d_sout_ = static_cast<float*>(alloc(static_cast<size_t>(Q_) * N_ * 4));
+bool Domain::form_dst_planes() {
+  if (a_buf_ < 0) return false;
   StepArgs a = args(false);
-  a.s_out = d_sout_;
+  a.s_out = planes_scratch();
   // planes only: read the buffer as-is (no moments written)
   check(launch_readback(lattice_, storage_, true, a, buf_[a_buf_], stream_), "readback");
-  h_fdst_.resize(static_cast<size_t>(Q_) * N_);
-  check(hipMemcpyAsync(h_fdst_.data(), d_sout_, h_fdst_.size() * 4, hipMemcpyDeviceToHost, stream_), "d2h");
-  check(hipStreamSynchronize(stream_), "readback");
+  fsrc_valid_ = sout_is_fsrc_ = false;  // d_sout_ now holds f_dst
+  return true;
+}
+
+const float* Domain::f_dst() {
+  if (fdst_valid_) return h_fdst_.data();
+  if (form_dst_planes()) {
+    h_fdst_.resize(static_cast<size_t>(Q_) * N_);
+    device_to_host(h_fdst_.data(), d_sout_, h_fdst_.size() * sizeof(float), stream_);
+  } else {
+    h_fdst_.assign(f_src(), f_src() + static_cast<size_t>(Q_) * N_);
+  }
   fdst_valid_ = true;
-  fsrc_valid_ = false;  // d_sout_ now holds f_dst
-  sout_is_fsrc_ = false;
   return h_fdst_.data();
 }
 
+void Domain::read_f_dst(float* out) {
+  const size_t bytes = static_cast<size_t>(Q_) * N_ * sizeof(float);
+  if (fdst_valid_) std::memcpy(out, h_fdst_.data(), bytes);
+  else if (form_dst_planes()) device_to_host(out, d_sout_, bytes, stream_);
+  else read_f_src(out);
+}
+
 void Domain::diagnostics(double out[3]) {
-  ensure_fields();
+  ensure_device_fields();
   sync_device_config();  // the reduction reads the device cell types
   check(launch_diagnostics(d_flags_, d_rho_, d_speed_, static_cast<long long>(N_), d_partial_, 1024, d_out_, stream_),
         "diagnostics");
@@ -1389,7 +1389,7 @@ void Domain::enable_thermal(float tau_g, float gbeta, float t_ref, float t_init)
     for (int k = 0; k < 2; ++k) gbuf_[k] = static_cast<float*>(alloc(5 * static_cast<size_t>(stride_) * sizeof(float)));
     d_twall_ = static_cast<float*>(alloc(N_ * sizeof(float)));
     d_temp_ = static_cast<float*>(alloc(N_ * sizeof(float)));
-    h_temp_.assign(N_, 0.0f);
+    check(hipMemsetAsync(d_temp_, 0, N_ * sizeof(float), stream_), "temperature");
   }
   h_twall_.assign(N_, std::numeric_limits<float>::quiet_NaN());
   twall_dirty_ = true;
@@ -1411,7 +1411,8 @@ void Domain::set_temperature_field(const float* t) {
     check(hipMemcpyAsync(gbuf_[k], host.data(), host.size() * sizeof(float), hipMemcpyHostToDevice, stream_),
           "upload temperature");
   check(hipStreamSynchronize(stream_), "upload temperature");
-  fields_valid_ = dfields_valid_ = false;
+  dfields_valid_ = false;
+  mirrors_ = 0;
 }
 
 void Domain::set_wall_temperature(int x0, int y0, int x1, int y1, float t_wall) {
@@ -1424,8 +1425,7 @@ void Domain::set_wall_temperature(int x0, int y0, int x1, int y1, float t_wall) 
 
 const float* Domain::temperature() {
   if (!thermal_) throw HipError("temperature is not enabled on this domain");
-  ensure_fields();
-  return h_temp_.data();
+  return mirror(5);
 }
 
 // ------------------------------------------------------------ batched steps

@@ -184,6 +184,14 @@ class Domain {
   // them adiabatic again.
   void set_wall_temperature(int x0, int y0, int x1, int y1, float t_wall);
   const float* temperature();
+  // One field into caller memory: 0 rho, 1 ux, 2 uy, 3 uz, 4 |u|, 5 the
+  // temperature (N floats); the populations S_k or A_{k-1} (Q N floats); an
+  // analytics field.  Straight from the device where no host mirror of it is
+  // current: only what is asked for crosses the bus, and once.
+  void read_field(int which, float* out);
+  void read_f_src(float* out);
+  void read_f_dst(float* out);
+  void read_analytics(int which, float* out);
   const float* thermal_buffer(int k) const { return gbuf_[k]; }
 
   // --- batched stepping (batch_host.cpp)
@@ -208,10 +216,16 @@ class Domain {
   void before_config_change();
   void materialize();
   void sync_device_config();
-  void ensure_fields();
-  void upload_state_from_host(const std::vector<float>& f_ref);
+  float* device_array(int which);       // the moment arrays and the temperature
+  const float* mirror(int which);       // host mirror of one of them, refreshed
+  void ensure_analytics(int which);     // device analytics arrays current
+  bool form_dst_planes();               // A_{k-1} planes into d_sout_ (false: no step yet)
+  void state_set();
+  float* planes_scratch();  // Q planes of N floats (d_sout_)
+  void form_planes();       // S_k into them
   void invalidate_mirrors() {
-    fields_valid_ = dfields_valid_ = fsrc_valid_ = fdst_valid_ = an_valid_ = false;
+    dfields_valid_ = fsrc_valid_ = fdst_valid_ = an_valid_ = false;
+    mirrors_ = an_mirrors_ = 0;
     sout_is_fsrc_ = false;
   }
   void ensure_device_fields();
@@ -348,16 +362,18 @@ class Domain {
   // analytics outputs (allocated on first use)
   float* d_an_[4] = {nullptr, nullptr, nullptr, nullptr};
   std::vector<float> h_an_[4];
-  bool an_valid_ = false;
-  std::vector<float> h_twall_, h_temp_;
+  bool an_valid_ = false;     // device analytics arrays current
+  unsigned an_mirrors_ = 0;   // bit k: h_an_[k] current
+  std::vector<float> h_twall_;
   bool twall_dirty_ = false;
 
   // host mirrors
-  std::vector<float> h_rho_, h_ux_, h_uy_, h_uz_, h_speed_, h_fsrc_, h_fdst_;
+  std::vector<float> h_field_[6], h_fsrc_, h_fdst_;  // fields: as read_field()'s numbers
   std::vector<float> h_prev_;  // staging of the outlet store (kept until the upload completes)
-  bool fields_valid_ = false, fsrc_valid_ = false, fdst_valid_ = false;
+  unsigned mirrors_ = 0;  // bit k: h_field_[k] current
+  bool fsrc_valid_ = false, fdst_valid_ = false;
   bool sout_is_fsrc_ = false;  // d_sout_ holds the bytes of the current f_src() mirror
-  bool dfields_valid_ = false;  // device moment arrays current (implied by fields_valid_)
+  bool dfields_valid_ = false;  // device moment arrays current
 };
 
 // splitmix64 finaliser (same constants as the device inlet turbulence).

@@ -153,6 +153,17 @@ hipError_t launch_materialize_thermal(const StepArgs& a, const float* g_in, floa
 // rho, u (with the node's buoyancy in the Guo shift), |u| and T of S_k.
 hipError_t launch_readback_thermal(int storage, bool from_s, const StepArgs& a, const void* buf,
                                    const float* gbuf, hipStream_t s);
+// State from fields (FP32 device arrays; uz unused in 2D): feq of every node
+// in storage format into buf, |u| into speed, the outlet records into prev
+// (state_init.hip, the host expressions' rounding).
+hipError_t launch_init_fields(int lattice, int storage, const float* rho, const float* ux, const float* uy,
+                              const float* uz, float* speed, void* buf, long long stride, float* prev, int nx, int N,
+                              hipStream_t s);
+// State from FP32 planes of N values, plus seeded noise U(-a, a) of counter
+// node * Q + q when amplitude is not zero.
+hipError_t launch_init_planes(int lattice, int storage, const float* planes, float amplitude,
+                              unsigned long long seed, void* buf, long long stride, float* prev, int nx, int N,
+                              hipStream_t s);
 // Materialise S_k (commit=true updates the convective outlet store) into
 // s_state (storage format, stride a.stride), or fields/planes for read-back.
 hipError_t launch_materialize(int lattice, int storage, const StepArgs& a, const void* a_in, void* s_state,
