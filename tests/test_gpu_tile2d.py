@@ -130,3 +130,38 @@ def test_force_history_over_mixed_steps(wa):
         assert first == 0 and f.shape == (216, 3) and np.array_equal(f[:81], mid)
         hist.append(f)
     assert np.array_equal(*hist)
+
+
+@pytest.mark.parametrize("storage", [0, 1, 2])
+@pytest.mark.parametrize("scene,chunk,graph", [("channel", 7, True), ("noisy", 16, False), ("lid", 100, True),
+                                               ("cavity", 6, True)])
+def test_batch_tiles_equal_single_steps(wa, scene, chunk, graph, storage):
+    """A batch takes tile launches where all its members may: members of
+    several sizes with their own step counts (ends inside a launch, chunks
+    that are no multiple of a launch, a graph that is replayed) keep the bits
+    and the forces of single-step launches, and can be stepped on alone."""
+    make, kinds, forces = SCENES[scene]
+    coll, les = kinds[0]
+    sizes, steps = [(240, 80), (33, 17), (16, 16), (64, 33)], [5, 12, 43, 8]
+    ends = []
+    for multi in (True, False):
+        grids = [make(wa, nx, ny, storage) for nx, ny in sizes]
+        for g in grids:
+            g.set_multistep(multi)
+            if les or scene in ("channel", "noisy"):
+                g.set_les_coupled(les)
+        b = wa.Batch(lattice=9, storage=storage, collision=coll, use_les=les, chunk=chunk, thermal=forces is None)
+        ids = [b.add(g, k, g=(1e-6, -1e-6, 0.0), smag=0.17,
+                     forces=(nx / 3.0, ny / 2.0, 0.0, 0.0) if forces else None)
+               for g, k, (nx, ny) in zip(grids, steps, sizes)]
+        b.run(20, use_graph=graph)
+        b.run(30, use_graph=graph)
+        end = [b.forces(i) for i in ids]
+        assert not forces or [len(f) for f in end] == steps
+        for i, g in zip(ids, grids):
+            b.remove(i)
+            g.run(3, coll, use_les=les, smag=0.17)
+            end += _state(g, forces is None)
+        ends.append(end)
+    for a, c in zip(*ends):
+        assert np.array_equal(a, c, equal_nan=True)

@@ -41,7 +41,8 @@ HOST_FLAGS = ["-O2", "-std=c++20", "-fPIC", "-ffp-contract=off", f"--offload-arc
               "-Wno-unused-command-line-argument"]
 
 SOURCES = [
-    "step_d3q19.hip", "step_d3q27.hip", "step_d2q9.hip", "tile2d.hip", "step_kernels.hip", "thermal.hip", "analytics.hip",
+    "step_d3q19.hip", "step_d3q27.hip", "step_d2q9.hip", "tile2d.hip", "tile2d_batch.hip",
+    "step_kernels.hip", "thermal.hip", "analytics.hip",
     "ispc_compat.hip", "batch.hip", "domain.cpp", "capi.cpp", "lattice_grid.cpp", "runner.cpp", "batch_host.cpp",
     "host_api.cpp", "host_pipe.cpp", "geometry.hip", "state_init.hip", "export.cpp", "thermal_solver.cpp", "hbm_probe.hip",
 ]

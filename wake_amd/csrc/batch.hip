@@ -103,14 +103,14 @@ __global__ __launch_bounds__(256) void k_mem_batch(const BatchSlot* __restrict__
   }
 }
 
-__global__ void k_advance_batch(BatchSlot* __restrict__ slots, int nslots, int k) {
+__global__ void k_advance_batch(BatchSlot* __restrict__ slots, int nslots, int k, int span) {
   const int s = blockIdx.x * blockDim.x + threadIdx.x;
   if (s >= nslots) return;
   BatchSlot& sl = slots[s];
   const unsigned long long left = sl.stop_at > sl.step ? sl.stop_at - sl.step : 0ull;
   const unsigned long long taken = left < static_cast<unsigned long long>(k) ? left : static_cast<unsigned long long>(k);
   sl.step += taken;
-  sl.parity = (sl.parity + static_cast<int>(taken & 1ull)) & 1;
+  sl.parity = (sl.parity + static_cast<int>((taken + span - 1) / span)) & 1;
 }
 
 namespace {
@@ -213,9 +213,10 @@ hipError_t launch_mem_batch(int lattice, int storage, const BatchSlot* slots, in
   }
 }
 
-hipError_t launch_advance_batch(BatchSlot* slots, int nslots, int k, hipStream_t s) {
+hipError_t launch_advance_batch(BatchSlot* slots, int nslots, int k, int span, hipStream_t s) {
   if (nslots <= 0) return hipSuccess;
-  k_advance_batch<<<(nslots + 255) / 256, 256, 0, s>>>(slots, nslots, k);
+  if (span < 1) return hipErrorInvalidValue;
+  k_advance_batch<<<(nslots + 255) / 256, 256, 0, s>>>(slots, nslots, k, span);
   return hipGetLastError();
 }
 

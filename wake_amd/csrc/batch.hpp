@@ -35,6 +35,10 @@ struct BatchSlot {
   const int* mem_nodes;
   int mem_count;
   int mem_on;                 // forces recorded for this member
+  // tile launches (2D): tiles [ttile0, ..) in rows of ttiles_x, and where the
+  // tiles leave the sums of the nodes in mem_nodes
+  int ttile0, ttiles_x;
+  TileForces tile_forces;
 };
 
 // One launch = step i of the chunk for every slot.  grid_x work-groups of
@@ -49,7 +53,20 @@ hipError_t launch_step_batch(int lattice, int storage, int collision, bool les, 
 // hist[(slot * chunk + i) * 3 + k].  Slots past their stop step are skipped.
 hipError_t launch_mem_batch(int lattice, int storage, const BatchSlot* slots, int nslots, int i, int chunk,
                             double* hist, hipStream_t s);
-// End of a chunk of `k` launches: step += steps taken, parity updated.
-hipError_t launch_advance_batch(BatchSlot* slots, int nslots, int k, hipStream_t s);
+// End of a chunk of `k` steps, `span` steps a launch: step += steps taken,
+// parity updated (once per launch taken).
+hipError_t launch_advance_batch(BatchSlot* slots, int nslots, int k, int span, hipStream_t s);
+// 2D members without curved links and convective outlets: the steps i .. i +
+// nsteps - 1 of the chunk (nsteps <= span, 8 or 4) in one launch, the
+// flip-th of the chunk (tile2d_batch.hip); force: some member has a body
+// force.
+hipError_t launch_tile2d_batch(int storage, int collision, bool les, bool thermal, bool force, int span,
+                               const BatchSlot* slots, const int* tile_slot, int ntiles, int i, int flip, int nsteps,
+                               hipStream_t s);
+// The forces after those steps, hist as in launch_mem_batch.
+hipError_t launch_mem_tiles(int storage, const BatchSlot* slots, int nslots, int i, int flip, int nsteps, int chunk,
+                            double* hist, hipStream_t s);
+// Tiles of an nx x ny domain with `span` steps a launch.
+void tile2d_grid(int nx, int ny, int span, int* tiles_x, int* tiles);
 
 }  // namespace wake_hip

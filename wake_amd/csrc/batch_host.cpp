@@ -332,6 +332,8 @@ class Batch {
     drop_graph();
     const int n = static_cast<int>(members_.size());
     if (!shape_explicit_) shape_.block = default_block();
+    span_ = pick_span();
+    any_g_ = false;
     std::vector<BatchSlot> slots(n);
     std::vector<int> tile_slot;
     any_forces_ = false;
@@ -355,9 +357,18 @@ class Batch {
       b.tile0 = static_cast<int>(tile_slot.size());
       b.tiles_per_row = (m.d->nx() + shape_.block - 1) / shape_.block;
       b.ntiles = m.d->ny() * m.d->nz() * b.tiles_per_row;
-      tile_slot.insert(tile_slot.end(), b.ntiles, s);
+      if (span_ > 1) {
+        b.ttile0 = static_cast<int>(tile_slot.size());
+        int tiles = 0;
+        tile2d_grid(m.d->nx(), m.d->ny(), span_, &b.ttiles_x, &tiles);
+        tile_slot.insert(tile_slot.end(), tiles, s);
+      } else {
+        tile_slot.insert(tile_slot.end(), b.ntiles, s);
+      }
+      any_g_ = any_g_ || b.a.gx != 0.0f || b.a.gy != 0.0f;
       if (m.forces) {
         b.mem_nodes = m.d->batch_mem_nodes(m.c[0], m.c[1], m.c[2], m.r_max, &b.mem_count);
+        if (span_ > 1) b.tile_forces = m.d->batch_tile_forces();
         b.mem_on = 1;
         b.a.mem_c[0] = m.c[0];
         b.a.mem_c[1] = m.c[1];
@@ -396,6 +407,23 @@ class Batch {
     layout_dirty_ = false;
   }
 
+  // Steps a launch: 2D members that all may take tile launches do (the rule
+  // and the sizes of Domain::tile_eligible, over the batch's nodes); a launch
+  // shape then has no effect.
+  int pick_span() const {
+    if (lattice_ != 9 || members_.empty()) return 1;
+    const bool one_per_unit = thermal_ && storage_ == kStoreF32;
+    long long tiles = 0;
+    for (const auto& m : members_) {
+      if (!m.d->batch_tiles()) return 1;
+      int tx = 0, t = 0;
+      tile2d_grid(m.d->nx(), m.d->ny(), kTbSteps, &tx, &t);
+      tiles += t;
+    }
+    if (!Domain::tiles_pay(storage_, thermal_, nodes())) return 1;
+    return tile2d_steps_for(tiles, one_per_unit);
+  }
+
   int grid_x() const {
     if (shape_.grid_factor == 0) return ntiles_;
     return std::min(ntiles_, shape_.grid_factor * cus_);
@@ -403,13 +431,25 @@ class Batch {
 
   void enqueue_chunk(int k) {
     const int n = static_cast<int>(members_.size());
+    if (span_ > 1) {
+      for (int i = 0, flip = 0; i < k; i += span_, ++flip) {
+        const int steps = std::min(span_, k - i);
+        check(launch_tile2d_batch(storage_, collision_, les_, thermal_, any_g_, span_, d_slots_, d_tiles_, ntiles_, i,
+                                  flip, steps, stream_),
+              "batch tiles");
+        if (any_forces_)
+          check(launch_mem_tiles(storage_, d_slots_, n, i, flip, steps, chunk_, d_hist_, stream_), "batch forces");
+      }
+      check(launch_advance_batch(d_slots_, n, k, span_, stream_), "batch advance");
+      return;
+    }
     for (int i = 0; i < k; ++i) {
       check(launch_step_batch(lattice_, storage_, collision_, les_, thermal_, buf_ok_, d_slots_, d_tiles_, ntiles_, i,
                               shape_.block, grid_x(), stream_),
             "batch step");
       if (any_forces_) check(launch_mem_batch(lattice_, storage_, d_slots_, n, i, chunk_, d_hist_, stream_), "batch forces");
     }
-    check(launch_advance_batch(d_slots_, n, k, stream_), "batch advance");
+    check(launch_advance_batch(d_slots_, n, k, 1, stream_), "batch advance");
   }
 
   void capture() {
@@ -455,7 +495,7 @@ class Batch {
           m.hist.insert(m.hist.end(), o, o + 3);
         }
       m.step += taken;
-      m.parity = (m.parity + static_cast<int>(taken & 1)) & 1;
+      m.parity = (m.parity + static_cast<int>((taken + span_ - 1) / span_)) & 1;
     }
   }
 
@@ -482,6 +522,8 @@ class Batch {
   bool layout_dirty_ = true;
   bool any_forces_ = false;
   bool buf_ok_ = true;
+  bool any_g_ = false;  // some member has a body force
+  int span_ = 1;        // steps a launch (more than 1: tile launches)
   bool pending_ = false;
   int pending_k_ = 0;
   BatchSlot* d_slots_ = nullptr;

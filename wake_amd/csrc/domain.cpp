@@ -710,13 +710,16 @@ void Domain::materialize() {
 }
 
 // ------------------------------------------------------------------ step
-bool Domain::tile_eligible() const {
+bool Domain::tile_kind() const {
   if (dim_ != 2 || !tile_enabled_) return false;
   // curved links and the convective outlet read past the tile's halo
   if (n_bfl_nodes_ > 0 || outflow_ == 2) return false;
   // (the temperature kernels with BF16 storage round some products otherwise
   // in a step loop than in a single step)
-  if (thermal_ && storage_ == kStoreBF16) return false;
+  return !(thermal_ && storage_ == kStoreBF16);
+}
+
+bool Domain::tiles_pay(int storage, bool thermal, uint64_t nodes) {
   // Measured, us a step of single launches / tiles: FP32 channels 4.4 / 1.7 at
   // 240 x 80, 13.2 / 8.3 at 1500 x 403, 202 / 147 at 4096^2; FP32 temperature
   // 6.1 / 2.1 at 240 x 80, 36 / 31 at 1536 x 1024, 341 / 326 at 4096^2.  With
@@ -724,8 +727,15 @@ bool Domain::tile_eligible() const {
   // domains do without: TRT channels 19.2 / 19.7 at 1536 x 1024, 151 / 153 at
   // 4096^2 (MRT 135 / 130); temperature 14.3 / 13.7 at 1024 x 512, 30 / 37 at
   // 1536 x 1024.
-  if (storage_ == kStoreF32) return true;
-  return N_ <= (thermal_ ? 1u << 19 : 1u << 23);
+  if (storage == kStoreF32) return true;
+  return nodes <= (thermal ? 1u << 19 : 1u << 23);
+}
+
+bool Domain::tile_eligible() const { return tile_kind() && tiles_pay(storage_, thermal_, N_); }
+
+bool Domain::batch_tiles() {
+  sync_device_config();
+  return tile_kind();
 }
 
 bool Domain::plain_periodic() const {
@@ -1469,12 +1479,28 @@ const int* Domain::batch_mem_nodes(float ccx, float ccy, float ccz, float r_max,
       release(d_batch_nodes_);
       d_batch_nodes_ = nullptr;
     }
+    if (d_batch_index_ || d_batch_sums_) check(hipStreamSynchronize(stream_), "batch nodes");
+    release(d_batch_index_);
+    release(d_batch_sums_);
+    d_batch_index_ = nullptr;
+    d_batch_sums_ = nullptr;
     batch_rows_ = build_mem_rows(ccx, ccy, ccz, r_max);
     batch_rows_key_ = key;
     d_batch_nodes_ = build_mem_nodes(batch_rows_, ccx, ccy, ccz, r_max, &n_batch_nodes_);
   }
   *count = n_batch_nodes_;
   return d_batch_nodes_;
+}
+
+TileForces Domain::batch_tile_forces() {
+  if (n_batch_nodes_ > 0 && !d_batch_index_) {
+    d_batch_index_ = static_cast<int*>(alloc(N_ * sizeof(int)));
+    d_batch_sums_ = static_cast<double*>(alloc(3 * sizeof(double) * kTbSteps * static_cast<size_t>(n_batch_nodes_)));
+    check(hipMemsetAsync(d_batch_index_, 0xff, N_ * sizeof(int), stream_), "batch nodes");
+    check(launch_index_nodes(d_batch_nodes_, n_batch_nodes_, d_batch_index_, stream_), "batch nodes");
+    check(hipStreamSynchronize(stream_), "batch nodes");  // the batch runs on its own stream
+  }
+  return TileForces{d_batch_index_, d_batch_sums_, n_batch_nodes_, kTbSteps};
 }
 
 size_t Domain::bytes_needed(int dim, int lattice, int nx, int ny, int nz, int storage, long long plane_pad,

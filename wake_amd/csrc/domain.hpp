@@ -92,7 +92,12 @@ class Domain {
   void step(int collision, float gx, float gy, float gz, bool use_les, float smag);
   // run() takes up to kTbSteps steps per launch where tile_eligible() (2D
   // domains); off: one launch per step.
-  void set_multistep(bool on) { tile_enabled_ = on; }
+  void set_multistep(bool on) {
+    tile_enabled_ = on;
+    ++version_;
+  }
+  // Whether tile launches beat single steps for `nodes` 2D nodes.
+  static bool tiles_pay(int storage, bool thermal, uint64_t nodes);
   // `steps` steps; returns the device time in ms measured with events on the
   // domain's stream around the launches.
   float run(int steps, int collision, float gx, float gy, float gz, bool use_les, float smag, bool timed);
@@ -207,6 +212,11 @@ class Domain {
   // r_max, in node order: a device list the domain owns (valid until the
   // next call or a geometry change), *count entries.
   const int* batch_mem_nodes(float cx, float cy, float cz, float r_max, int* count);
+  // Whether this domain may take tile launches in a batch (its size aside).
+  bool batch_tiles();
+  // Where tile launches of a batch leave the sums of batch_mem_nodes() (a
+  // ring of kTbSteps steps).
+  TileForces batch_tile_forces();
   // Device bytes a domain of this shape allocates.
   static size_t bytes_needed(int dim, int lattice, int nx, int ny, int nz, int storage, long long plane_pad = -1,
                              bool thermal = false);
@@ -298,6 +308,7 @@ class Domain {
   uint8_t* d_flags_ = nullptr;
   uint8_t* d_cls_ = nullptr;
   uint32_t* d_bmask_ = nullptr;  // per node: bounce mask of the kClsSlow nodes
+  bool tile_kind() const;        // 2D without curved links or convective outlet, not switched off
   bool tile_eligible() const;
   bool plain_periodic() const;   // no node carries a class bit
   bool all_fluid_ = false;       // every cell type Fluid (set with the class bytes)
@@ -324,6 +335,8 @@ class Domain {
   MemRows batch_rows_;  // the rows of batch_mem_nodes(), with their key
   int* d_batch_nodes_ = nullptr;
   int n_batch_nodes_ = 0;
+  int* d_batch_index_ = nullptr;     // node -> its place in d_batch_nodes_, or -1
+  double* d_batch_sums_ = nullptr;   // kTbSteps x n_batch_nodes_ x 3
   std::tuple<float, float, float, float, uint64_t> batch_rows_key_{0.0f, 0.0f, 0.0f, 0.0f, ~0ull};
   double* d_mempart_ = nullptr;  // partials of one momentum_exchange() call
   size_t mempart_cap_ = 0;       // in doubles

@@ -109,6 +109,7 @@ inline int mem_waves_per_row(int nx) { return (nx + 63) / 64; }
 hipError_t launch_build_class(int lattice, const StepArgs& a, uint8_t* cls, uint32_t* bmask, hipStream_t s);
 // Most steps of one tile launch (launch_tile2d): the halo of its LDS tiles.
 inline constexpr int kTbSteps = 8;
+inline constexpr int kTbFewSteps = 4;  // of one on domains of many tiles
 // Where a tile launch writes the force sums (3 doubles) of the nodes holding
 // momentum-exchange links: node n's sum of step k goes to
 // out[3 ((k % ring) count + index[n]) ..]; index[n] is -1 for other nodes.
@@ -122,6 +123,7 @@ struct TileForces {
 // Steps a tile launch of such a domain takes best (at most kTbSteps);
 // one_per_unit: a compute unit holds one of its tiles (FP32 temperature).
 int tile2d_steps_of(int nx, int ny, bool one_per_unit);
+int tile2d_steps_for(long long tiles_of_most, bool one_per_unit);  // the rule, by tiles of kTbSteps steps
 // nsteps (at most kTbSteps) steps of a 2D domain without curved links and
 // without the convective outlet, from A_{k-1} in `in` (from_s: from a
 // materialised S_k, the first step collides only) to A_{k-1+nsteps} in `out`;

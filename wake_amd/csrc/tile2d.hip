@@ -67,7 +67,7 @@ __global__ __launch_bounds__(256) void k_index_nodes(const int* __restrict__ nod
 namespace {
 
 // Tiles of W x H nodes with a halo of T own (W - 2 T) x (H - 2 T).
-constexpr int kTileW = 32, kTileH = 32, kTileLowH = 24, kTileFewSteps = 4;
+constexpr int kTileW = 32, kTileH = 32, kTileLowH = 24;
 
 template <int T, int W, int H>
 dim3 tiles_of(int nx, int ny) {
@@ -107,12 +107,12 @@ hipError_t go(const StepArgs& a, const void* in, void* out, const float* gin, fl
     return hipGetLastError();
   };
   using Many = std::integral_constant<int, kTbSteps>;
-  using Few = std::integral_constant<int, kTileFewSteps>;
+  using Few = std::integral_constant<int, kTbFewSteps>;
   using High = std::integral_constant<int, kTileH>;
   using Low = std::integral_constant<int, kTileLowH>;
   auto sized = [&](auto force, auto edge) {
     constexpr bool one_per_unit = THERMAL && sizeof(T_) == 4;
-    if (nsteps <= kTileFewSteps && tile2d_steps_of(a.nx, a.ny, one_per_unit) == kTileFewSteps)
+    if (nsteps <= kTbFewSteps && tile2d_steps_of(a.nx, a.ny, one_per_unit) == kTbFewSteps)
       return run(force, edge, Few{}, High{});
     if (low_tiles(a)) return run(force, edge, Many{}, Low{});
     return run(force, edge, Many{}, High{});
@@ -154,9 +154,12 @@ hipError_t go_collision(int collision, bool les, const StepArgs& a, const void* 
 // 512 x 256 nodes (512 tiles of 8 steps) 3.60 / 3.85, 768 x 384 (1152)
 // 6.70 / 5.27; temperature FP32 256 x 256 (256 tiles) 2.87 / 4.19, 512 x 256
 // 5.31 / 4.43.
+int tile2d_steps_for(long long tiles_of_most, bool one_per_unit) {
+  return tiles_of_most <= (one_per_unit ? 1ll : 2ll) * compute_units() ? kTbSteps : kTbFewSteps;
+}
 int tile2d_steps_of(int nx, int ny, bool one_per_unit) {
   const dim3 g = tiles_of<kTbSteps, kTileW, kTileH>(nx, ny);
-  return static_cast<long long>(g.x) * g.y <= (one_per_unit ? 1ll : 2ll) * compute_units() ? kTbSteps : kTileFewSteps;
+  return tile2d_steps_for(static_cast<long long>(g.x) * g.y, one_per_unit);
 }
 
 hipError_t launch_tile2d(int storage, int collision, bool les, bool thermal, bool from_s, bool edges, int nsteps,
