@@ -18,6 +18,7 @@
 #include "wake_hip.h"
 #include "domain.hpp"
 #include "engine.hpp"
+#include "host_pipe.hpp"
 #include "lattice.hpp"
 #include "node_ops.hpp"
 
@@ -96,11 +97,14 @@ class Call {
   }
   bool end() {
     if (hipGetLastError() != hipSuccess) return fail("kernel launch");
-    if (hipDeviceSynchronize() != hipSuccess) return fail("kernel");
-    for (auto& r : regions_)
-      if (r.copy_out && r.host && r.bytes)
-        if (hipMemcpy(r.host, g_stage.base() + r.offset, r.bytes, hipMemcpyDeviceToHost) != hipSuccess)
-          return fail("hipMemcpy D2H");
+    if (hipStreamSynchronize(nullptr) != hipSuccess) return fail("kernel");
+    try {
+      for (auto& r : regions_)
+        if (r.copy_out && r.host && r.bytes) device_to_host(r.host, g_stage.base() + r.offset, r.bytes, nullptr);
+    } catch (const std::exception& e) {
+      record_error(std::string("wake: ") + name_ + ": " + e.what());
+      return false;
+    }
     return true;
   }
 
@@ -456,7 +460,7 @@ void collide_call(const char* name, const float* f_in, float* f_out, const uint8
   Call c(name);
   const size_t n = static_cast<size_t>(count);
   auto fi = c.in(f_in, L::Q * n);
-  auto fo = c.inout(f_out, L::Q * n);
+  auto fo = c.out(f_out, L::Q * n);  // every element is written (solid nodes copy)
   auto t = c.in(ct, n);
   auto r = c.inout(rho, n);
   auto a = c.inout(ux, n);
