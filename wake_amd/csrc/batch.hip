@@ -53,20 +53,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(StepWaves<L
       else m = collide<L, COLL, false, St::kFast>(f, a.tau, a.gx, a.gy, a.gz);
       flag_nonfinite(a, m.rho);
     }
-    if constexpr (St::kBuf) {
-      const auto r = St::rsrc(out, static_cast<unsigned>(L::Q * a.stride * sizeof(T)));
-      static_for<L::Q>([&](auto qc) {
-        constexpr int q = decltype(qc)::value;
-        St::template stb<L, q>(r, static_cast<unsigned>(x) * sizeof(T),
-                               static_cast<unsigned>(q * a.stride + static_cast<long long>(row) * a.nx) * sizeof(T),
-                               f[q]);
-      });
-    } else {
-      static_for<L::Q>([&](auto qc) {
-        constexpr int q = decltype(qc)::value;
-        St::template st<L, q>(out, q * a.stride + n, f[q]);
-      });
-    }
+    store_node<L, St>(a, out, x, static_cast<long long>(row) * a.nx, f);
   }
 }
 

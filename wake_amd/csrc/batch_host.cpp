@@ -380,6 +380,11 @@ class Batch {
       m.parity = parity;
       m.seen_version = m.d->version();
     }
+    // the members' buffers share the caches
+    unsigned long long bytes = 0;
+    for (const BatchSlot& b : slots)
+      bytes += 2ull * lattice_ * b.a.stride * (storage_ == kStoreF32 ? 4ull : 2ull);
+    for (BatchSlot& b : slots) b.a.keep_stores = keep_stores_for(bytes) ? 1 : 0;
     ntiles_ = static_cast<int>(tile_slot.size());
     if (n > slot_cap_) {
       if (d_slots_) (void)hipFree(d_slots_);

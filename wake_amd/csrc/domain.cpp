@@ -612,12 +612,14 @@ StepArgs Domain::args(bool commit) const {
   a.bz0 = dim_ == 2 ? 0 : (a.per_z ? 0 : 1);
   a.bz1 = dim_ == 2 ? 1 : (a.per_z ? nz_ : nz_ - 1);
   a.commit_prev = commit ? 1 : 0;
+  a.keep_stores = keep_stores_for(2ull * Q_ * stride_ * elem_) ? 1 : 0;
   a.global_addr = buffer_addressing_ ? 0 : 1;
   a.f_prev = d_prev_;
   a.flags = d_flags_;
   a.cls = d_cls_;
   a.aux = d_aux_;
   a.bmask = d_bmask_;
+  a.mmask = d_mmask_;
   a.bfl = d_bfl_;
   a.gx = g_last_[0];
   a.gy = g_last_[1];
@@ -686,8 +688,10 @@ void Domain::sync_device_config() {
   }
   if (cls_dirty_) {
     all_fluid_ = std::all_of(flags_.begin(), flags_.end(), [](uint8_t t) { return t == kFluid; });
+    if (!d_mmask_ && std::find(flags_.begin(), flags_.end(), static_cast<uint8_t>(kMovingWall)) != flags_.end())
+      d_mmask_ = static_cast<uint32_t*>(alloc(N_ * sizeof(uint32_t)));
     const StepArgs a = args(false);
-    check(launch_build_class(lattice_, a, d_cls_, d_bmask_, stream_), "build class");
+    check(launch_build_class(lattice_, a, d_cls_, d_bmask_, d_mmask_, stream_), "build class");
     check(launch_mark_bfl(d_bfl_nodes_, n_bfl_nodes_, d_cls_, d_aux_, stream_), "mark bfl");
     cls_dirty_ = false;
     ++cls_epoch_;

@@ -308,6 +308,7 @@ class Domain {
   uint8_t* d_flags_ = nullptr;
   uint8_t* d_cls_ = nullptr;
   uint32_t* d_bmask_ = nullptr;  // per node: bounce mask of the kClsSlow nodes
+  uint32_t* d_mmask_ = nullptr;  // per node: moving-wall directions (allocated with the first moving wall)
   bool tile_kind() const;        // 2D without curved links or convective outlet, not switched off
   bool tile_eligible() const;
   bool plain_periodic() const;   // no node carries a class bit

@@ -51,6 +51,10 @@ struct BflNode {
 
 struct StepArgs {
   int nx, ny, nz;
+  // population stores stay in the caches (keep_stores_for); here so that it
+  // is loaded with the sizes: a scalar load of its own just before the stores
+  // holds every wave up (0.3 us of a 64^3 step)
+  int keep_stores;
   long long stride;          // population plane stride in elements (>= nx*ny*nz)
   int periodic_mode;         // reference stream_periodic: the pull ignores cell types
   int per_y, per_z;          // boundary mode: wrap y / z instead of reflecting
@@ -77,6 +81,7 @@ struct StepArgs {
   const uint8_t* cls;         // ClassBits
   const int* aux;             // per node: index into bfl[] (valid where kClsBfl)
   const uint32_t* bmask;      // per node: bounce mask (valid where kClsSlow); null: from the cell types
+  const uint32_t* mmask;      // per node: directions whose pull source is a MovingWall (valid where kBounceMovingWall)
   const BflNode* bfl;
   // read-back outputs
   float* rho;
@@ -102,11 +107,26 @@ struct StepArgs {
   int* nonfinite;
 };
 
+// Whether the populations of a step should stay in the caches after their
+// store.  Non-temporal stores leave them to memory, which is right for
+// buffers larger than the 256 MB last-level cache (4 % at 256^3 FP32) and for
+// small ones, where the write-back of dirty lines at the launch's end adds
+// about a microsecond; between, the next step reads what this one wrote from
+// the cache.  Measured, us a step non-temporal / cached, both buffers' MB:
+// 61 x 45 x 37 FP32 (15) 12.1 / 13.9; 64^3 FP16 (20) 9.7 / 11.0; 64^3 FP32
+// (40) 10.5 / 11.5 with open boundaries, 10.5 / 9.5 periodic; 96^3 FP16 (67)
+// 22.0 / 18.6; 96^3 FP32 (134) 29.9 / 25.8; 128^3 FP16 (159) 36.9 / 29.0;
+// 160 x 128 x 112 FP16 (174) 56.5 / 53.4; 128^3 FP32 (319) 62.3 / 63.6;
+// 192^3 FP16 (538) 112 / 117.
+inline bool keep_stores_for(unsigned long long both_buffers) {
+  return both_buffers >= (48ull << 20) && both_buffers <= (240ull << 20);
+}
+
 // Partial slots of one force sample: rows with links x waves per row.
 inline int mem_waves_per_row(int nx) { return (nx + 63) / 64; }
 
 // Launchers (step_kernels.hip).  `lattice` is 9, 19 or 27.
-hipError_t launch_build_class(int lattice, const StepArgs& a, uint8_t* cls, uint32_t* bmask, hipStream_t s);
+hipError_t launch_build_class(int lattice, const StepArgs& a, uint8_t* cls, uint32_t* bmask, uint32_t* mmask, hipStream_t s);
 // Most steps of one tile launch (launch_tile2d): the halo of its LDS tiles.
 inline constexpr int kTbSteps = 8;
 inline constexpr int kTbFewSteps = 4;  // of one on domains of many tiles

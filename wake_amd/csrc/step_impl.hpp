@@ -50,13 +50,15 @@ namespace wake_hip {
 #define WAKE_NT_STORES 1
 #endif
 
-template <class T>
+template <bool KEEP = false, class T>
 __device__ __forceinline__ void st_pop(T* __restrict__ p, long long i, T v) {
 #if WAKE_NT_STORES
-  __builtin_nontemporal_store(v, p + i);
-#else
-  p[i] = v;
+  if constexpr (!KEEP) {
+    __builtin_nontemporal_store(v, p + i);
+    return;
+  }
 #endif
+  p[i] = v;
 }
 
 template <class T>
@@ -78,8 +80,8 @@ struct StF32 {
   __device__ __forceinline__ static float ld(const T* __restrict__ p, long long i) {
     return ld_pop(p, i);
   }
-  template <class L, int q>
-  __device__ __forceinline__ static void st(T* __restrict__ p, long long i, float v) { st_pop(p, i, v); }
+  template <class L, int q, bool KEEP = false>
+  __device__ __forceinline__ static void st(T* __restrict__ p, long long i, float v) { st_pop<KEEP>(p, i, v); }
 };
 
 // FP16 <-> FP32 with the weight offset in one mixed-precision FMA each:
@@ -112,9 +114,9 @@ struct StF16 {
   __device__ __forceinline__ static float ld(const T* __restrict__ p, long long i) {
     return f16_bits_plus(__builtin_bit_cast(unsigned short, ld_pop(p, i)), L::w[q]);
   }
-  template <class L, int q>
+  template <class L, int q, bool KEEP = false>
   __device__ __forceinline__ static void st(T* __restrict__ p, long long i, float v) {
-    st_pop(p, i, __builtin_bit_cast(_Float16, f16_bits_of_minus(v, L::w[q])));
+    st_pop<KEEP>(p, i, __builtin_bit_cast(_Float16, f16_bits_of_minus(v, L::w[q])));
   }
   template <class L, int q>
   __device__ __forceinline__ static float from_dev_bits(unsigned short h) {
@@ -142,9 +144,9 @@ struct StBF16 {
   __device__ __forceinline__ static float ld(const T* __restrict__ p, long long i) {
     return L::w[q] + __uint_as_float(static_cast<uint32_t>(ld_pop(p, i)) << 16);
   }
-  template <class L, int q>
+  template <class L, int q, bool KEEP = false>
   __device__ __forceinline__ static void st(T* __restrict__ p, long long i, float v) {
-    st_pop(p, i, static_cast<uint16_t>(to_bits(v - L::w[q])));
+    st_pop<KEEP>(p, i, static_cast<uint16_t>(to_bits(v - L::w[q])));
   }
   template <class L, int q>
   __device__ __forceinline__ static float from_dev_bits(unsigned short h) {
@@ -179,14 +181,15 @@ struct StBuf : Base {
       return Base::template from_dev_bits<L, q>(h);
     }
   }
-  template <class L, int q>
+  template <class L, int q, bool KEEP = false>
   __device__ __forceinline__ static void stb(__amdgpu_buffer_rsrc_t r, unsigned voff, unsigned soff, float v) {
+    constexpr int kPolicy = KEEP ? 0 : kNonTemporal;
     if constexpr (sizeof(typename Base::T) == 4) {
       __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v), r, static_cast<int>(voff), static_cast<int>(soff),
-                                            kNonTemporal);
+                                            kPolicy);
     } else {
       __builtin_amdgcn_raw_buffer_store_b16(Base::template dev_bits<L, q>(v), r, static_cast<int>(voff),
-                                            static_cast<int>(soff), kNonTemporal);
+                                            static_cast<int>(soff), kPolicy);
     }
   }
 };
@@ -319,16 +322,21 @@ __device__ __forceinline__ void gather(const StepArgs& a, const typename St::T* 
       return 2.0f * L::w[q] * 1.0f * 3.0f * ci_uw;
     };
     if (a.bmask) {
-      // the bounce mask built with the class bytes: no cell-type reads
+      // the masks built with the class bytes: no cell-type reads (read per
+      // direction next to a moving wall, each before the population it belongs
+      // to, they took 1.1 of 12 us a step in a 61 x 45 x 37 lid-driven box)
       const uint32_t bm = a.bmask[n];
+      const uint32_t moving = (bm & kBounceMovingWall) ? a.mmask[n] : 0u;
       static_for<L::Q>([&](auto qc) {
         constexpr int q = decltype(qc)::value;
         if constexpr (q > 0) {
           if (bm & (1u << q)) {
             float v = St::template ld<L, L::opp[q]>(A, L::opp[q] * S + n);
-            if (bm & kBounceMovingWall) {
-              bool in;
-              if (source(qc, in) == kMovingWall) v += moving_wall_term(qc);
+            if (moving & (1u << q)) {
+              // (the mark keeps this a branch: as a select it would make
+              // every bouncing direction wait for its own load)
+              asm volatile("; moving wall");
+              v += moving_wall_term(qc);
             }
             f[q] = v;
           }
@@ -716,16 +724,48 @@ __device__ __forceinline__ void mem_wave(const StepArgs& a, bool want, int x, in
   }
 }
 
+// A node's populations into the output buffer (x: its column, row: the first
+// node of its row), kept in the caches or past them as the launch asks.
+template <class L, class St, bool KEEP>
+__device__ __forceinline__ void store_node_as(const StepArgs& a, typename St::T* __restrict__ out, int x,
+                                              long long row, const float (&f)[L::Q]) {
+  const long long S = a.stride;
+  // (the marks keep the two kinds of stores apart: hoisted or merged out of
+  // the two branches, they would lose the non-temporal bit)
+  if constexpr (KEEP) asm volatile("; cached stores");
+  if constexpr (St::kBuf) {
+    const auto r = St::rsrc(out, static_cast<unsigned>(L::Q * S * sizeof(typename St::T)));
+    constexpr unsigned E = sizeof(typename St::T);
+    static_for<L::Q>([&](auto qc) {
+      constexpr int q = decltype(qc)::value;
+      St::template stb<L, q, KEEP>(r, static_cast<unsigned>(x) * E, static_cast<unsigned>(q * S + row) * E, f[q]);
+    });
+  } else {
+    static_for<L::Q>([&](auto qc) {
+      constexpr int q = decltype(qc)::value;
+      St::template st<L, q, KEEP>(out, q * S + row + x, f[q]);
+    });
+  }
+  if constexpr (KEEP) asm volatile("; end of cached stores");
+}
+template <class L, class St>
+__device__ __forceinline__ void store_node(const StepArgs& a, typename St::T* __restrict__ out, int x, long long row,
+                                           const float (&f)[L::Q]) {
+  if (a.keep_stores) store_node_as<L, St, true>(a, out, x, row, f);
+  else store_node_as<L, St, false>(a, out, x, row, f);
+}
+
 // ----------------------------------------------------------------- kernels
 template <class L>
-__global__ void k_build_class(const StepArgs a, uint8_t* __restrict__ cls, uint32_t* __restrict__ bmask) {
+__global__ void k_build_class(const StepArgs a, uint8_t* __restrict__ cls, uint32_t* __restrict__ bmask,
+                              uint32_t* __restrict__ mmask) {
   const int x = blockIdx.x * blockDim.x + threadIdx.x;
   const int y = blockIdx.y, z = blockIdx.z;
   if (x >= a.nx) return;
   const int n = (z * a.ny + y) * a.nx + x;
   const uint8_t t = a.flags[n];
   uint8_t c = 0;
-  uint32_t mask = 0;
+  uint32_t mask = 0, moving = 0;
   if (t == kSolid) c |= a.periodic_mode ? kClsSolid : (kClsSolid | kClsFrozen);
   if (!a.periodic_mode && t != kSolid) {
     if (t == kFluid) mask |= kBounceFluid;
@@ -742,13 +782,15 @@ __global__ void k_build_class(const StepArgs a, uint8_t* __restrict__ cls, uint3
         else {
           const uint8_t nt = a.flags[(sz * a.ny + sy) * a.nx + sx];
           if (nt == kSolid || nt == kMovingWall) mask |= 1u << q;
-          if (nt == kMovingWall) mask |= kBounceMovingWall;
+          if (nt == kMovingWall) moving |= 1u << q;
         }
       }
     });
+    if (moving) mask |= kBounceMovingWall;
     if (mask & ~kBounceFluid) c |= kClsSlow;
   }
   if (bmask) bmask[n] = mask;
+  if (mmask) mmask[n] = moving;
   const bool in_rows = y >= a.by0 && y < a.by1 && z >= a.bz0 && z < a.bz1;
   if (a.inflow && x == 0 && in_rows) c |= kClsInlet;
   if (a.outflow && x == a.nx - 1 && in_rows) c |= kClsOutlet;
@@ -867,20 +909,7 @@ __global__ __launch_bounds__(256) WAKE_STEP_ATTR void k_step(const StepArgs a, c
       else m = collide<L, COLL, false, St::kFast>(f, a.tau, a.gx, a.gy, a.gz);
       flag_nonfinite(a, m.rho);
     }
-    if constexpr (St::kBuf) {
-      const auto r = St::rsrc(aout, static_cast<unsigned>(L::Q * S * sizeof(typename St::T)));
-      constexpr unsigned E = sizeof(typename St::T);
-      const long long row = static_cast<long long>((z * a.ny + y) * a.nx);
-      static_for<L::Q>([&](auto qc) {
-        constexpr int q = decltype(qc)::value;
-        St::template stb<L, q>(r, static_cast<unsigned>(x) * E, static_cast<unsigned>(q * S + row) * E, f[q]);
-      });
-    } else {
-      static_for<L::Q>([&](auto qc) {
-        constexpr int q = decltype(qc)::value;
-        St::template st<L, q>(aout, q * S + n, f[q]);
-      });
-    }
+    store_node<L, St>(a, aout, x, static_cast<long long>((z * a.ny + y) * a.nx), f);
   }
 }
 

@@ -79,11 +79,12 @@ __global__ __launch_bounds__(256) void k_diag_final(const double* __restrict__ p
   }
 }
 
-hipError_t launch_build_class(int lattice, const StepArgs& a, uint8_t* cls, uint32_t* bmask, hipStream_t s) {
+hipError_t launch_build_class(int lattice, const StepArgs& a, uint8_t* cls, uint32_t* bmask, uint32_t* mmask,
+                              hipStream_t s) {
   switch (lattice) {
-    case 9: return detail::build_class_d2q9(a, cls, bmask, s);
-    case 19: return detail::build_class_d3q19(a, cls, bmask, s);
-    case 27: return detail::build_class_d3q27(a, cls, bmask, s);
+    case 9: return detail::build_class_d2q9(a, cls, bmask, mmask, s);
+    case 19: return detail::build_class_d3q19(a, cls, bmask, mmask, s);
+    case 27: return detail::build_class_d3q27(a, cls, bmask, mmask, s);
     default: return hipErrorInvalidValue;
   }
 }

@@ -113,16 +113,7 @@ __device__ __forceinline__ void tile2d_steps(Tile2dShared<St, THERMAL, W, H>& sh
     else in = sy >= 0 && sy < ny;
     return in ? sy * nx + sx : n;
   };
-  if (bm & kBounceMovingWall) {
-    static_for<L::Q>([&](auto qc) {
-      constexpr int q = decltype(qc)::value;
-      if constexpr (q > 0) {
-        bool in;
-        const int sn = source(L::cx[q], L::cy[q], in);
-        if (in && ap->flags[sn] == kMovingWall) moving |= 1u << q;
-      }
-    });
-  }
+  if (bm & kBounceMovingWall) moving = ap->mmask[n];
   if constexpr (THERMAL) {
     if (c & kClsSlow) {
       static_for<D2Q5::Q>([&](auto qc) {
