@@ -165,3 +165,37 @@ def test_batch_tiles_equal_single_steps(wa, scene, chunk, graph, storage):
         ends.append(end)
     for a, c in zip(*ends):
         assert np.array_equal(a, c, equal_nan=True)
+
+
+def _warm_cavity(wa, nx, ny, storage):
+    """Side walls at temperatures whose product with 2 w rounds."""
+    g = _cavity(wa, nx, ny, storage)
+    g.set_wall_temperature(0, 0, 0, ny - 1, 0.87)
+    g.set_wall_temperature(nx - 1, 0, nx - 1, ny - 1, 0.21)
+    return g
+
+
+def _same_as_single_steps(wa, make, nx, ny, storage, coll, les=False, gx=0.0, gy=0.0, thermal=False, probe=False,
+                          runs=(1, 3, 8, 2, 21)):
+    ends = []
+    for multi in (True, False):
+        g = make(wa, nx, ny, storage)
+        g.set_multistep(multi)
+        if probe:
+            g.set_force_probe(nx / 3.0, ny / 2.0, 0.0, 0.0)
+        for steps in runs:
+            g.run(steps, coll, gx=gx, gy=gy, use_les=les, smag=0.17)
+        end = _state(g, thermal) + [g.f_dst_data().copy()]
+        if probe:
+            end.append(g.force_history()[1])
+        ends.append(end)
+    for k, (a, b) in enumerate(zip(*ends)):
+        assert np.array_equal(a, b, equal_nan=True), k
+
+
+@pytest.mark.parametrize("coll", ["BGK", "TRT", "MRT"])
+@pytest.mark.parametrize("storage", [0, 1])
+@pytest.mark.parametrize("nx,ny", [(33, 17), (131, 8), (240, 80), (256, 256)])
+def test_wall_temperatures_in_tiles(wa, nx, ny, storage, coll):
+    """The anti-bounce-back term 2 w T_wall keeps the single step's rounding."""
+    _same_as_single_steps(wa, _warm_cavity, nx, ny, storage, coll, gx=1e-6, gy=-2e-6, thermal=True)

@@ -60,6 +60,9 @@ __device__ __forceinline__ TileArgs* opaque_args(TileArgs* p) {
   return p;
 }
 
+// The same value, as one the compiler knows nothing of.
+__device__ __forceinline__ void opaque(float& v) { asm volatile("" : "+v"(v)); }
+
 // Steps s_step + 1 .. s_step + nsteps (nsteps <= T, the tile's halo) of the
 // tile whose own nodes start at (ox, oy).  from_s: `ain` holds a materialised S, the
 // first step only collides.  mf: where the own nodes' force sums go
@@ -103,7 +106,7 @@ __device__ __forceinline__ void tile2d_steps(Tile2dShared<St, THERMAL, W, H>& sh
   }
   if (!(c & kClsSlow)) bm = 0;
   uint32_t moving = 0;  // directions whose pull source is a moving wall
-  float t_wall[D2Q5::Q];
+  float t_wall[D2Q5::Q] = {};
   uint32_t g_wall = 0;  // temperature directions whose pull source reflects
   auto source = [&](int cx, int cy, bool& in) {
     const int sx = wrap(x - cx, nx);
@@ -190,6 +193,12 @@ __device__ __forceinline__ void tile2d_steps(Tile2dShared<St, THERMAL, W, H>& sh
     }
     if constexpr (FORCE || THERMAL) asm volatile("" : "+s"(b.gx), "+s"(b.gy));
     if constexpr (THERMAL) asm volatile("" : "+s"(b.gbeta), "+s"(b.t_ref));
+    if constexpr (THERMAL && EDGE) {
+      static_for<D2Q5::Q>([&](auto qc) {
+        constexpr int q = decltype(qc)::value;
+        if constexpr (q > 0) opaque(t_wall[q]);  // 2 w T_wall is such a product
+      });
+    }
     if (i >= s && i < W - s && j >= s && j < H - s) {
       float f[L::Q];
       const bool pull = !(from_s && s == 1) && !(EDGE && (c & kClsFrozen));
