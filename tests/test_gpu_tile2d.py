@@ -199,3 +199,33 @@ def _same_as_single_steps(wa, make, nx, ny, storage, coll, les=False, gx=0.0, gy
 def test_wall_temperatures_in_tiles(wa, nx, ny, storage, coll):
     """The anti-bounce-back term 2 w T_wall keeps the single step's rounding."""
     _same_as_single_steps(wa, _warm_cavity, nx, ny, storage, coll, gx=1e-6, gy=-2e-6, thermal=True)
+
+
+def _thick_channel(wa, nx, ny, storage, turb=False):
+    """Solid nodes inside the inlet and outlet rows: walls two nodes thick, a
+    step at the inlet and a sill at the outlet."""
+    g = _channel(wa, nx, ny, storage, turb)
+    g.set_solid_box(0, 1, nx - 1, 1)
+    g.set_solid_box(0, ny - 3, min(4, nx // 3), ny - 2)
+    g.set_solid_box(nx - 2, ny // 2, nx - 1, ny // 2)
+    return g
+
+
+@pytest.mark.parametrize("storage", [0, 1, 2])
+@pytest.mark.parametrize("coll,les,turb", [("MRT", True, False), ("TRT", False, True)])
+@pytest.mark.parametrize("nx,ny", [(240, 80), (33, 17), (17, 48), (9, 8)])
+def test_solid_nodes_on_open_boundaries(wa, nx, ny, coll, les, turb, storage):
+    """Their post-collision populations take the closures as in a single step."""
+    _same_as_single_steps(wa, lambda *a: _thick_channel(*a, turb=turb), nx, ny, storage, coll, les, probe=True)
+
+
+def test_solid_nodes_on_open_boundaries_of_a_cavity(wa):
+    def make(wa, nx, ny, storage):
+        g = _thick_channel(wa, nx, ny, storage)
+        g.set_les_coupled(False)
+        g.enable_thermal(0.62, 1e-3, 0.5, 0.5)
+        g.set_temperature_field(np.random.default_rng(1).uniform(0, 1, nx * ny).astype(np.float32))
+        g.set_wall_temperature(0, 0, nx - 1, 1, 0.87)
+        return g
+
+    _same_as_single_steps(wa, make, 64, 33, 0, "MRT", thermal=True)
