@@ -229,3 +229,32 @@ def test_solid_nodes_on_open_boundaries_of_a_cavity(wa):
         return g
 
     _same_as_single_steps(wa, make, 64, 33, 0, "MRT", thermal=True)
+
+
+@pytest.mark.parametrize("read", [False, True])
+@pytest.mark.parametrize("gap", [1, 10, 100])
+def test_force_history_around_batch_steps(wa, gap, read):
+    """A batch takes no probe samples: the history ends where it stood, and
+    later runs add none of steps that were not sampled."""
+    hist = []
+    for multi in (True, False):
+        g = _channel(wa, 150, 50, 0)
+        g.set_multistep(multi)
+        g.set_force_probe(50.0, 25.0, 0.0, 20.0)
+        g.run(20, "MRT", use_les=True, smag=0.17)
+        before = g.force_history()[1].copy() if read else None
+        b = wa.Batch(lattice=9, collision="MRT", use_les=True)
+        slot = b.add(g, gap, smag=0.17)
+        b.run(gap)
+        b.remove(slot)
+        g.run(30, "MRT", use_les=True, smag=0.17)
+        first, f = g.force_history()
+        assert first == 0 and (before is None or np.array_equal(f[:len(before)], before))
+        # read at step 20, sample 20 is there, and a batch of one step leaves no gap
+        assert len(f) == (20 + 1 + 30 + 1 if read and gap == 1 else 21 if read else 20)
+        g.set_force_probe(50.0, 25.0, 0.0, 20.0)
+        g.run(9, "MRT", use_les=True, smag=0.17)
+        hist.append((f, g.force_history()[1]))
+        assert len(hist[-1][1]) == 10
+    for a, b in zip(*hist):
+        assert np.array_equal(a, b)

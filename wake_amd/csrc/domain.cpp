@@ -750,7 +750,10 @@ void Domain::step_tile(int nsteps, int collision, float gx, float gy, bool use_l
   version_ += static_cast<uint64_t>(nsteps);
   const bool from_s = s_buf_ >= 0;
   TileForces mf{};
-  if (probe_) {
+  // samples follow one another: after steps that took none (a batch's) the
+  // history stays where it ended
+  const bool sampling = probe_ && fh_next_ >= step_count_;
+  if (sampling) {
     probe_sync();
     // a launch from a materialised S forms S_{k+1} first
     if (from_s) probe_sample_current();
@@ -774,7 +777,7 @@ void Domain::step_tile(int nsteps, int collision, float gx, float gy, bool use_l
   g_last_[1] = gy;
   g_last_[2] = 0.0f;
   step_count_ += static_cast<uint64_t>(nsteps);
-  if (probe_) fh_next_ = tile_end_ = step_count_;
+  if (sampling) fh_next_ = tile_end_ = step_count_;
   invalidate_mirrors();
 }
 
