@@ -122,3 +122,38 @@ def test_diagnostics_and_analytics_without_host_fields(wa):
     wa.kernels.kernel("compute_vorticity_and_q_criterion_3d", *u, ox, oy, oz, qc, 61, 33, 20)
     for a, b in zip(w, (ox, oy, oz, qc)):
         assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("storage", [0, 1])
+@pytest.mark.parametrize("steps", [0, 1, 2, 3, 8, 9, 16, 21])
+@pytest.mark.parametrize("op", ["populations", "noise", "fields", "uniform"])
+def test_temperature_goes_on_from_a_new_flow_state(wa, op, steps, storage):
+    """Setting the flow leaves the temperature where it is, whichever buffer
+    the steps before ended in, one launch per step or several."""
+    ends = []
+    nx, ny = 40, 27
+    for multi in (True, False):
+        g = wa.LatticeGrid2D(nx, ny, 0.6, storage=storage)
+        g.initialize(1.0)
+        g.set_solid_box(0, 0, nx - 1, 0)
+        g.set_solid_box(0, ny - 1, nx - 1, ny - 1)
+        g.enable_thermal(0.62, 1e-3, 0.5, 0.5)
+        g.set_temperature_field(np.random.default_rng(2).uniform(0, 1, nx * ny).astype(np.float32))
+        g.set_wall_temperature(0, 0, nx - 1, 0, 0.87)
+        g.set_multistep(multi)
+        g.run(steps, "MRT")
+        t0 = g.temperature_data().copy()
+        if op == "populations":
+            g.set_populations(g.f_src_data().copy())
+        elif op == "noise":
+            g.add_noise(1e-4, 5)
+        elif op == "fields":
+            g.initialize_fields(*_fields((nx, ny, 1), 9))
+        else:
+            g.initialize(1.0, 0.01, 0.0)
+        g.update_macroscopic()
+        assert np.array_equal(g.temperature_data(), t0)
+        g.run(3, "MRT")
+        ends.append([g.temperature_data().copy(), g.f_src_data().copy()])
+    for a, b in zip(*ends):
+        assert np.array_equal(a, b)

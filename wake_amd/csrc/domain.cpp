@@ -192,6 +192,7 @@ const void* Domain::state_buffer() const { return buf_[s_buf_ >= 0 ? s_buf_ : a_
 void Domain::initialize(float rho, float ux, float uy, float uz) {
   ++version_;
   const LatTab L = tab(lattice_);
+  const int slot = state_slot();
   if (dim_ == 2) uz = 0.0f;
   step_count_ = 0;
   const float u_sq = dim_ == 2 ? ux * ux + uy * uy : ux * ux + uy * uy + uz * uz;
@@ -201,7 +202,7 @@ void Domain::initialize(float rho, float ux, float uy, float uz) {
                                  : static_cast<float>(L.cx[q]) * ux + static_cast<float>(L.cy[q]) * uy +
                                        static_cast<float>(L.cz[q]) * uz;
     const float fe = L.w[q] * rho * (1.0f + 3.0f * ci_u + 4.5f * ci_u * ci_u - 1.5f * u_sq);
-    void* plane = static_cast<char*>(buf_[0]) + static_cast<size_t>(q) * stride_ * elem_;
+    void* plane = static_cast<char*>(buf_[slot]) + static_cast<size_t>(q) * stride_ * elem_;
     if (storage_ == kStoreF32) {
       uint32_t bits;
       std::memcpy(&bits, &fe, 4);
@@ -213,7 +214,7 @@ void Domain::initialize(float rho, float ux, float uy, float uz) {
     fe_q[q] = fe;
   }
   upload_prev([&](size_t, int q) { return fe_q[q]; });
-  s_buf_ = 0;
+  s_buf_ = slot;
   a_buf_ = -1;
   std::fill(flags_.begin(), flags_.end(), static_cast<uint8_t>(kFluid));
   flags_dirty_ = cls_dirty_ = true;
@@ -235,11 +236,22 @@ void Domain::initialize(float rho, float ux, float uy, float uz) {
   if (probe_) probe_restart();
 }
 
-// The state now is a materialised S in buffer 0, formed on the device.
-void Domain::state_set() {
+// The buffer a new state is written to.  A temperature goes on from where it
+// is: a materialised S of it lies in that slot when this returns.
+int Domain::state_slot() {
+  if (!thermal_) return 0;
+  if (s_buf_ >= 0) return s_buf_;
+  sync_device_config();
+  const int out = 1 - a_buf_;
+  check(launch_materialize_thermal(args(false), gbuf_[a_buf_], gbuf_[out], stream_), "materialize temperature");
+  return out;
+}
+
+// The state now is a materialised S in buffer `slot`, formed on the device.
+void Domain::state_set(int slot) {
   ++version_;
   clear_nonfinite();
-  s_buf_ = 0;
+  s_buf_ = slot;
   a_buf_ = -1;
   fsrc_valid_ = fdst_valid_ = sout_is_fsrc_ = false;
   if (probe_) probe_restart();  // the state the samples were taken of is gone
@@ -253,6 +265,7 @@ float* Domain::planes_scratch() {
 // lattice_grid_3d.cpp:95-131 with the per-node values as arrays; cell types
 // are left untouched.
 void Domain::initialize_fields(const float* rho, const float* ux, const float* uy, const float* uz) {
+  const int slot = state_slot();
   step_count_ = 0;
   float* dst[4] = {d_rho_, d_ux_, d_uy_, d_uz_};
   const float* src[4] = {rho, ux, uy, dim_ == 2 ? nullptr : uz};
@@ -260,10 +273,10 @@ void Domain::initialize_fields(const float* rho, const float* ux, const float* u
     if (src[k]) check(hipMemcpyAsync(dst[k], src[k], N_ * sizeof(float), hipMemcpyHostToDevice, stream_), "upload");
     else check(hipMemsetAsync(dst[k], 0, N_ * sizeof(float), stream_), "upload");
   }
-  check(launch_init_fields(lattice_, storage_, d_rho_, d_ux_, d_uy_, d_uz_, d_speed_, buf_[0], stride_, d_prev_, nx_,
-                           static_cast<int>(N_), stream_),
+  check(launch_init_fields(lattice_, storage_, d_rho_, d_ux_, d_uy_, d_uz_, d_speed_, buf_[slot], stride_, d_prev_,
+                           nx_, static_cast<int>(N_), stream_),
         "initialize");
-  state_set();
+  state_set(slot);
   check(hipStreamSynchronize(stream_), "upload");  // the caller's arrays are free again
   mirrors_ = 0;
   dfields_valid_ = true;  // the fields given, not the moments of their equilibria
@@ -271,13 +284,14 @@ void Domain::initialize_fields(const float* rho, const float* ux, const float* u
 
 void Domain::set_populations(const float* f_ref) {
   before_config_change();
+  const int slot = state_slot();
   check(hipMemcpyAsync(planes_scratch(), f_ref, static_cast<size_t>(Q_) * N_ * sizeof(float), hipMemcpyHostToDevice,
                        stream_),
         "upload");
-  check(launch_init_planes(lattice_, storage_, d_sout_, 0.0f, 0, buf_[0], stride_, d_prev_, nx_, static_cast<int>(N_),
-                           stream_),
+  check(launch_init_planes(lattice_, storage_, d_sout_, 0.0f, 0, buf_[slot], stride_, d_prev_, nx_,
+                           static_cast<int>(N_), stream_),
         "set populations");
-  state_set();
+  state_set(slot);
   check(hipStreamSynchronize(stream_), "upload");
   invalidate_mirrors();
 }
@@ -285,10 +299,11 @@ void Domain::set_populations(const float* f_ref) {
 // Seeded uniform noise U(-a, a) on every population, counter = node * Q + q.
 void Domain::add_noise(float amplitude, uint64_t seed) {
   form_planes();
-  check(launch_init_planes(lattice_, storage_, d_sout_, amplitude, seed, buf_[0], stride_, d_prev_, nx_,
+  const int slot = state_slot();
+  check(launch_init_planes(lattice_, storage_, d_sout_, amplitude, seed, buf_[slot], stride_, d_prev_, nx_,
                            static_cast<int>(N_), stream_),
         "noise");
-  state_set();
+  state_set(slot);
   check(hipStreamSynchronize(stream_), "noise");
 }
 

@@ -230,7 +230,8 @@ class Domain {
   const float* mirror(int which);       // host mirror of one of them, refreshed
   void ensure_analytics(int which);     // device analytics arrays current
   bool form_dst_planes();               // A_{k-1} planes into d_sout_ (false: no step yet)
-  void state_set();
+  int state_slot();
+  void state_set(int slot);
   float* planes_scratch();  // Q planes of N floats (d_sout_)
   void form_planes();       // S_k into them
   void invalidate_mirrors() {
