@@ -157,3 +157,41 @@ def test_temperature_goes_on_from_a_new_flow_state(wa, op, steps, storage):
         ends.append([g.temperature_data().copy(), g.f_src_data().copy()])
     for a, b in zip(*ends):
         assert np.array_equal(a, b)
+
+
+def _vorticity(wa, g, shape):
+    nx, ny, nz = shape
+    if nz == 1:
+        w = np.zeros(nx * ny, np.float32)
+        wa.kernels.kernel("compute_vorticity_2d", g.ux_data(), g.uy_data(), w, nx, ny)
+        return [w]
+    out = [np.zeros(nx * ny * nz, np.float32) for _ in range(4)]
+    wa.kernels.kernel("compute_vorticity_and_q_criterion_3d", g.ux_data(), g.uy_data(), g.uz_data(), *out, nx, ny, nz)
+    return out
+
+
+@pytest.mark.parametrize("lattice,shape", [(9, (53, 37, 1)), (19, (21, 17, 9))])
+def test_analytics_follow_a_new_state(wa, lattice, shape):
+    """Vorticity and Q read before a state was set are not given for it."""
+    g = _grid(wa, lattice, shape, 0)
+    read = (lambda: [g.vorticity_data()]) if lattice == 9 else g.vorticity_q_data
+    F = _fields(shape, lattice)
+
+    def check():
+        for a, b in zip(read(), _vorticity(wa, g, shape)):
+            assert np.array_equal(a, b)
+
+    def with_temperature():
+        g.enable_thermal(0.62, 1e-2, 0.5, 0.5)
+        g.run(2, "BGK", gx=1e-4, gy=2e-4)
+        read()
+        g.set_temperature_field(np.random.default_rng(4).uniform(0, 1, g.total_nodes()).astype(np.float32))
+
+    ops = [lambda: g.initialize_fields(*F), lambda: g.initialize(1.0, 0.02, 0.0),
+           lambda: g.initialize_fields(*[F[0]] + [np.float32(0.5) * u for u in F[1:]]),
+           lambda: g.run(3, "BGK", gx=1e-4, gy=2e-4), g.update_macroscopic, lambda: g.set_populations(g.f_src_data()),
+           lambda: g.add_noise(1e-3, 1)] + ([with_temperature] if lattice == 9 else [])
+    check()
+    for op in ops:
+        op()
+        check()

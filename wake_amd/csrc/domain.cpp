@@ -227,10 +227,8 @@ void Domain::initialize(float rho, float ux, float uy, float uz) {
     std::memcpy(&b, &vals[k], 4);
     check(hipMemsetD32Async(static_cast<hipDeviceptr_t>(dst[k]), b, N_, stream_), "fill");
   }
+  invalidate_mirrors();
   dfields_valid_ = true;
-  mirrors_ = 0;
-  fsrc_valid_ = fdst_valid_ = false;
-  sout_is_fsrc_ = false;
   clear_nonfinite();
   check(hipStreamSynchronize(stream_), "initialize");
   if (probe_) probe_restart();
@@ -278,7 +276,7 @@ void Domain::initialize_fields(const float* rho, const float* ux, const float* u
         "initialize");
   state_set(slot);
   check(hipStreamSynchronize(stream_), "upload");  // the caller's arrays are free again
-  mirrors_ = 0;
+  drop_fields();
   dfields_valid_ = true;  // the fields given, not the moments of their equilibria
 }
 
@@ -967,8 +965,7 @@ void Domain::read_field(int which, float* out) {
 void Domain::update_macroscopic() {
   const float keep[3] = {g_last_[0], g_last_[1], g_last_[2]};
   g_last_[0] = g_last_[1] = g_last_[2] = 0.0f;
-  dfields_valid_ = false;
-  mirrors_ = 0;
+  drop_fields();
   ensure_device_fields();
   g_last_[0] = keep[0];
   g_last_[1] = keep[1];
@@ -1443,8 +1440,7 @@ void Domain::set_temperature_field(const float* t) {
     check(hipMemcpyAsync(gbuf_[k], host.data(), host.size() * sizeof(float), hipMemcpyHostToDevice, stream_),
           "upload temperature");
   check(hipStreamSynchronize(stream_), "upload temperature");
-  dfields_valid_ = false;
-  mirrors_ = 0;
+  drop_fields();
 }
 
 void Domain::set_wall_temperature(int x0, int y0, int x1, int y1, float t_wall) {

@@ -234,10 +234,14 @@ class Domain {
   void state_set(int slot);
   float* planes_scratch();  // Q planes of N floats (d_sout_)
   void form_planes();       // S_k into them
-  void invalidate_mirrors() {
-    dfields_valid_ = fsrc_valid_ = fdst_valid_ = an_valid_ = false;
+  // the moments, and whatever was formed from them
+  void drop_fields() {
+    dfields_valid_ = an_valid_ = false;
     mirrors_ = an_mirrors_ = 0;
-    sout_is_fsrc_ = false;
+  }
+  void invalidate_mirrors() {
+    drop_fields();
+    fsrc_valid_ = fdst_valid_ = sout_is_fsrc_ = false;
   }
   void ensure_device_fields();
   void* alloc(size_t bytes);
