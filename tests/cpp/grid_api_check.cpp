@@ -12,6 +12,7 @@
 #include <sstream>
 #include <memory>
 #include <string>
+#include <thread>
 #include <vector>
 
 #include "wake_hip.h"
@@ -166,6 +167,88 @@ class GridScenario : public Scenario {
   LatticeGrid2D grid_;
   double mlups_ = 0.0;
 };
+
+// Pointers fetched once stay current, as a program that keeps them over its
+// steps expects (the reference's arrays are the grid's own).
+static void held_pointers() {
+  const int nx = 24, ny = 17, nz = 9;
+  LatticeGrid3D g(nx, ny, nz, 0.7f), h(nx, ny, nz, 0.7f);
+  const std::size_t n = g.total_nodes();
+  const real_t* held[5] = {g.rho_data(), g.ux_data(), g.uy_data(), g.uz_data(), g.speed_data()};
+  const auto flow = [](real_t scale) {
+    return [scale](int x, int y, int z, real_t& rho, real_t& ux, real_t& uy, real_t& uz) {
+      rho = 1.0f + 0.01f * std::sin(0.3f * x + 0.2f * z);
+      ux = scale * std::sin(0.4f * y);
+      uy = scale * std::cos(0.3f * z + 0.1f * x);
+      uz = scale * std::sin(0.2f * x + 0.5f * y);
+    };
+  };
+  // h takes the same calls and every pointer again each time
+  const auto same = [&](const char* what) {
+    const real_t* now[5] = {h.rho_data(), h.ux_data(), h.uy_data(), h.uz_data(), h.speed_data()};
+    for (int k = 0; k < 5; ++k)
+      EXPECT(std::memcmp(held[k], now[k], n * sizeof(real_t)) == 0, "held field %d after %s", k, what);
+  };
+  const auto both = [&](auto&& call) {
+    call(g);
+    call(h);
+  };
+  same("construction");
+  both([&](LatticeGrid3D& d) { d.initialize_custom(flow(0.03f)); });
+  same("initialize_custom");
+  for (int k = 0; k < 3; ++k) {
+    both([&](LatticeGrid3D& d) { d.step(CollisionType::BGK, 1e-5f, 0.0f, 2e-5f); });
+    g.update_macroscopic();
+    h.update_macroscopic();
+    same("update_macroscopic");
+  }
+  const auto step = [&] { both([&](LatticeGrid3D& d) { d.step(CollisionType::MRT, 1e-5f, 0.0f, 2e-5f); }); };
+  step();
+  EXPECT(g.uy_data() == held[2], "uy pointer");
+  same("uy_data()");
+  step();
+  (void)g.compute_total_mass();
+  same("compute_total_mass()");
+  step();
+  const real_t* f = g.f_src_data();
+  same("f_src_data()");
+  both([&](LatticeGrid3D& d) { d.add_noise(1e-3f, 7); });
+  same("add_noise");
+  EXPECT(std::memcmp(f, h.f_src_data(), 19 * n * sizeof(real_t)) == 0, "held f_src after add_noise");
+  both([&](LatticeGrid3D& d) { d.initialize_custom(flow(-0.02f)); });
+  same("a second initialize_custom");
+  EXPECT(std::memcmp(f, h.f_src_data(), 19 * n * sizeof(real_t)) == 0, "held f_src after initialize_custom");
+  both([&](LatticeGrid3D& d) { d.initialize(1.02f, 0.01f, 0.0f, -0.01f); });
+  same("initialize");
+  EXPECT(std::memcmp(f, h.f_src_data(), 19 * n * sizeof(real_t)) == 0, "held f_src after initialize");
+
+  LatticeGrid2D a(31, 20, 0.7f), b(31, 20, 0.7f);
+  const real_t* sp = a.speed_data();
+  for (LatticeGrid2D* d : {&a, &b}) {
+    d->initialize(1.0f, 0.03f, 0.01f);
+    d->set_solid_box(0, 0, 30, 0);
+    d->step(CollisionType::TRT);
+    d->update_macroscopic();
+  }
+  EXPECT(std::memcmp(sp, b.speed_data(), a.total_nodes() * sizeof(real_t)) == 0, "held 2D speed");
+
+  // first accesses from several threads at once
+  LatticeGrid3D t(nx, ny, nz, 0.7f);
+  t.initialize_custom(flow(0.03f));
+  t.step(CollisionType::BGK);
+  t.update_macroscopic();
+  double sums[8] = {};
+  std::vector<std::thread> threads;
+  for (int k = 0; k < 8; ++k)
+    threads.emplace_back([&, k] {
+      for (int z = 0; z < nz; ++z)
+        for (int y = 0; y < ny; ++y)
+          for (int x = 0; x < nx; ++x)
+            sums[k] += t.rho(x, y, z) + t.ux(x, y, z) + t.uy(x, y, z) + t.uz(x, y, z) + t.speed(x, y, z);
+    });
+  for (auto& th : threads) th.join();
+  for (int k = 1; k < 8; ++k) EXPECT(sums[k] == sums[0], "fields of thread %d", k);
+}
 
 static void runner() {
   auto sc = std::make_shared<GridScenario>();
@@ -595,6 +678,7 @@ int main(int argc, char** argv) {
     taylor_green_3d();
     poiseuille_2d();
     sphere_forces();
+    held_pointers();
     runner();
   } catch (const WakeException& e) {
     std::printf("FAIL: exception %s\n", e.what());

@@ -232,6 +232,7 @@ void Domain::initialize(float rho, float ux, float uy, float uz) {
   clear_nonfinite();
   check(hipStreamSynchronize(stream_), "initialize");
   if (probe_) probe_restart();
+  refresh_held();
 }
 
 // The buffer a new state is written to.  A temperature goes on from where it
@@ -253,6 +254,12 @@ void Domain::state_set(int slot) {
   a_buf_ = -1;
   fsrc_valid_ = fdst_valid_ = sout_is_fsrc_ = false;
   if (probe_) probe_restart();  // the state the samples were taken of is gone
+}
+
+// After a state was set: whatever of it was handed out before.
+void Domain::refresh_held() {
+  refresh_mirrors(0);
+  if (!h_fsrc_.empty()) f_src();
 }
 
 float* Domain::planes_scratch() {
@@ -278,6 +285,7 @@ void Domain::initialize_fields(const float* rho, const float* ux, const float* u
   check(hipStreamSynchronize(stream_), "upload");  // the caller's arrays are free again
   drop_fields();
   dfields_valid_ = true;  // the fields given, not the moments of their equilibria
+  refresh_held();
 }
 
 void Domain::set_populations(const float* f_ref) {
@@ -292,6 +300,7 @@ void Domain::set_populations(const float* f_ref) {
   state_set(slot);
   check(hipStreamSynchronize(stream_), "upload");
   invalidate_mirrors();
+  refresh_held();
 }
 
 // Seeded uniform noise U(-a, a) on every population, counter = node * Q + q.
@@ -303,6 +312,7 @@ void Domain::add_noise(float amplitude, uint64_t seed) {
         "noise");
   state_set(slot);
   check(hipStreamSynchronize(stream_), "noise");
+  refresh_held();
 }
 
 // ------------------------------------------------------------- cell types
@@ -942,18 +952,27 @@ float* Domain::device_array(int which) {
 }
 
 const float* Domain::mirror(int which) {
-  if (!(mirrors_ & (1u << which))) {
-    ensure_device_fields();
-    h_field_[which].resize(N_);
-    device_to_host(h_field_[which].data(), device_array(which), N_ * sizeof(float), stream_);
-    mirrors_ |= 1u << which;
-  }
+  if (!(mirrors_.load(std::memory_order_acquire) & (1u << which))) refresh_mirrors(1u << which);
   return h_field_[which].data();
+}
+
+void Domain::refresh_mirrors(unsigned want) {
+  std::lock_guard<std::mutex> lock(mirror_mutex_);
+  held_ |= want;
+  const unsigned stale = held_ & ~mirrors_.load(std::memory_order_relaxed);
+  if (stale == 0) return;
+  ensure_device_fields();
+  for (int k = 0; k < 6; ++k) {
+    if (!(stale & (1u << k))) continue;
+    h_field_[k].resize(N_);
+    device_to_host(h_field_[k].data(), device_array(k), N_ * sizeof(float), stream_);
+  }
+  mirrors_.fetch_or(stale, std::memory_order_release);
 }
 
 void Domain::read_field(int which, float* out) {
   if (which == 5 && !thermal_) throw HipError("temperature is not enabled on this domain");
-  if (mirrors_ & (1u << which)) {
+  if (mirrors_.load(std::memory_order_acquire) & (1u << which)) {
     std::memcpy(out, h_field_[which].data(), N_ * sizeof(float));
     return;
   }
@@ -967,6 +986,7 @@ void Domain::update_macroscopic() {
   g_last_[0] = g_last_[1] = g_last_[2] = 0.0f;
   drop_fields();
   ensure_device_fields();
+  refresh_mirrors(0);
   g_last_[0] = keep[0];
   g_last_[1] = keep[1];
   g_last_[2] = keep[2];
@@ -991,6 +1011,7 @@ void Domain::ensure_analytics(int which) {
 
 const float* Domain::analytics(int which) {
   ensure_analytics(which);
+  refresh_mirrors(0);
   if (!(an_mirrors_ & (1u << which))) {
     h_an_[which].resize(N_);
     device_to_host(h_an_[which].data(), d_an_[which], N_ * sizeof(float), stream_);
@@ -1040,6 +1061,7 @@ const float* Domain::f_src() {
   device_to_host(h_fsrc_.data(), d_sout_, h_fsrc_.size() * sizeof(float), stream_);
   fsrc_valid_ = true;
   sout_is_fsrc_ = true;
+  refresh_mirrors(0);
   return h_fsrc_.data();
 }
 
@@ -1086,6 +1108,7 @@ void Domain::read_f_dst(float* out) {
 
 void Domain::diagnostics(double out[3]) {
   ensure_device_fields();
+  refresh_mirrors(0);
   sync_device_config();  // the reduction reads the device cell types
   check(launch_diagnostics(d_flags_, d_rho_, d_speed_, static_cast<long long>(N_), d_partial_, 1024, d_out_, stream_),
         "diagnostics");

@@ -13,9 +13,11 @@
 
 #include <hip/hip_runtime.h>
 
+#include <atomic>
 #include <cstdint>
 #include <functional>
 #include <map>
+#include <mutex>
 #include <stdexcept>
 #include <string>
 #include <tuple>
@@ -107,7 +109,12 @@ class Domain {
   // stream; the open-boundary plane kernel is excluded).
   float last_kernel_ms() const { return last_kernel_ms_; }
 
-  // --- read-back (lazily synced host mirrors, reference layout)
+  // --- read-back (host mirrors in the reference layout).  A pointer stays
+  // good for the domain's life.  What the field pointers handed out point to
+  // is current after update_macroscopic(), after any call that gives a
+  // field, a diagnostic, analytics or populations, and after one that sets
+  // the state; f_src()'s after f_src() and after one that sets the state.
+  // Threads may call the field accessors together.
   const float* rho();
   const float* ux();
   const float* uy();
@@ -227,17 +234,20 @@ class Domain {
   void materialize();
   void sync_device_config();
   float* device_array(int which);       // the moment arrays and the temperature
-  const float* mirror(int which);       // host mirror of one of them, refreshed
+  const float* mirror(int which);       // host mirror of one of them, handed out
+  void refresh_mirrors(unsigned want);  // those of `want` and all handed out before
   void ensure_analytics(int which);     // device analytics arrays current
   bool form_dst_planes();               // A_{k-1} planes into d_sout_ (false: no step yet)
   int state_slot();
   void state_set(int slot);
+  void refresh_held();
   float* planes_scratch();  // Q planes of N floats (d_sout_)
   void form_planes();       // S_k into them
   // the moments, and whatever was formed from them
   void drop_fields() {
     dfields_valid_ = an_valid_ = false;
-    mirrors_ = an_mirrors_ = 0;
+    mirrors_.store(0, std::memory_order_relaxed);
+    an_mirrors_ = 0;
   }
   void invalidate_mirrors() {
     drop_fields();
@@ -389,7 +399,9 @@ class Domain {
   // host mirrors
   std::vector<float> h_field_[6], h_fsrc_, h_fdst_;  // fields: as read_field()'s numbers
   std::vector<float> h_prev_;  // staging of the outlet store (kept until the upload completes)
-  unsigned mirrors_ = 0;  // bit k: h_field_[k] current
+  std::atomic<unsigned> mirrors_{0};  // bit k: h_field_[k] current
+  unsigned held_ = 0;                 // bit k: h_field_[k] was handed out
+  std::mutex mirror_mutex_;
   bool fsrc_valid_ = false, fdst_valid_ = false;
   bool sout_is_fsrc_ = false;  // d_sout_ holds the bytes of the current f_src() mirror
   bool dfields_valid_ = false;  // device moment arrays current

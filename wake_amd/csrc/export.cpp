@@ -2,10 +2,10 @@
 // aerodynamic / performance telemetry as CSV and a JSON summary.
 //
 // src/export/vtk_exporter.cpp:8-223, src/export/csv_telemetry.cpp:8-127 and
-// src/forces/aerodynamic_telemetry.cpp:8-62.  The fields come from the
-// domain's host mirrors (one read-back kernel and one copy per field after
-// a step); the .vti is written either as the reference's ASCII text or as
-// one raw little-endian appended block per array.
+// src/forces/aerodynamic_telemetry.cpp:8-62.  The fields are read back once
+// per file (one kernel and one copy per field after a step); the .vti is
+// written either as the reference's ASCII text or as one raw little-endian
+// appended block per array.
 #include <algorithm>
 #include <cmath>
 #include <cstdint>
@@ -58,16 +58,16 @@ bool write_vti(Domain& d, const std::string& path, bool binary, const float* vor
   const int nx = d.nx(), ny = d.ny(), nz = d.nz();
   const size_t N = static_cast<size_t>(nx) * ny * nz;
   const bool three = d.dim() == 3;
-  const float *ux = d.ux(), *uy = d.uy(), *uz = three ? d.uz() : nullptr;
-  std::vector<float> vel(3 * N);
-  for (size_t i = 0; i < N; ++i) {
-    vel[3 * i] = ux[i];
-    vel[3 * i + 1] = uy[i];
-    vel[3 * i + 2] = three ? uz[i] : 0.0f;
+  std::vector<float> vel(3 * N, 0.0f), rho(N), speed(N);
+  for (int k = 0; k < (three ? 3 : 2); ++k) {
+    d.read_field(1 + k, speed.data());
+    for (size_t i = 0; i < N; ++i) vel[3 * i + k] = speed[i];
   }
+  d.read_field(4, speed.data());
+  d.read_field(0, rho.data());
   std::vector<PointArray> arrays = {{"Float32", "Velocity", 3, vel.data(), 4},
-                                    {"Float32", "Speed", 1, d.speed(), 4},
-                                    {"Float32", "Density", 1, d.rho(), 4}};
+                                    {"Float32", "Speed", 1, speed.data(), 4},
+                                    {"Float32", "Density", 1, rho.data(), 4}};
   if (!three && vort2d) arrays.push_back({"Float32", "Vorticity", 1, vort2d, 4});
   if (three && qcrit) arrays.push_back({"Float32", "Q_Criterion", 1, qcrit, 4});
   if (three && vort3d) arrays.push_back({"Float32", "Vorticity", 3, vort3d, 4});
