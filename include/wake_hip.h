@@ -240,7 +240,10 @@ int wake_domain_initialize(wake_domain* d, float rho, float ux, float uy, float 
  * arrays of nx*ny*nz (uz may be NULL) */
 int wake_domain_initialize_fields(wake_domain* d, const float* rho, const float* ux, const float* uy,
                                   const float* uz);
-/* Seeded uniform noise U(-a, a) on every population (counter = node*Q + q). */
+/* Seeded uniform noise U(-a, a) on every population (counter = node*Q + q).
+ * The fields read before the next step or update_macroscopic are those of
+ * the state without the noise; straight after wake_domain_set_populations
+ * with FP32 storage, those with it. */
 int wake_domain_add_noise(wake_domain* d, float amplitude, uint64_t seed);
 /* Replace the post-stream state by Q planes of nx*ny*nz (reference layout). */
 int wake_domain_set_populations(wake_domain* d, const float* f);

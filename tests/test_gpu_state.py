@@ -195,3 +195,39 @@ def test_analytics_follow_a_new_state(wa, lattice, shape):
     for op in ops:
         op()
         check()
+
+
+@pytest.mark.parametrize("storage", [0, 1])
+@pytest.mark.parametrize("lattice,shape", [(9, (53, 37, 1)), (19, (21, 17, 9))])
+def test_fields_after_noise(wa, lattice, shape, storage):
+    """They are those of the state without the noise until the next step,
+    whether or not a field was read before; FP32 planes just set have none."""
+    read = lambda g: [v.copy() for v in (g.rho_data(), g.ux_data(), g.uy_data(), g.speed_data())]
+
+    def stepped():
+        g = _grid(wa, lattice, shape, storage)
+        g.initialize_fields(*_fields(shape, lattice))
+        g.run(3, "BGK", gx=1e-4, gy=2e-4)
+        return g
+
+    clean = read(stepped())
+    for before in (lambda g: None, lambda g: g.rho_data(), lambda g: g.f_src_data(), lambda g: g.compute_max_speed()):
+        g = stepped()
+        before(g)
+        g.add_noise(1e-3, 8)
+        assert all(np.array_equal(a, b) for a, b in zip(read(g), clean))
+        g.add_noise(1e-3, 9)
+        assert all(np.array_equal(a, b) for a, b in zip(read(g), clean))
+        g.update_macroscopic()
+        assert not np.array_equal(g.rho_data(), clean[0])
+    g, h = stepped(), stepped()
+    f = g.f_src_data().copy()
+    for d in (g, h):
+        d.set_populations(f)
+    g.add_noise(1e-3, 8)
+    if storage:
+        want = read(h)
+    else:
+        h.set_populations(g.f_src_data().copy())
+        want = read(h)
+    assert all(np.array_equal(a, b) for a, b in zip(read(g), want))

@@ -300,11 +300,16 @@ void Domain::set_populations(const float* f_ref) {
   state_set(slot);
   check(hipStreamSynchronize(stream_), "upload");
   invalidate_mirrors();
+  planes_given_ = storage_ == kStoreF32;
   refresh_held();
 }
 
 // Seeded uniform noise U(-a, a) on every population, counter = node * Q + q.
+// The fields stay those of the state without it until the next step, except
+// right after set_populations() with FP32 storage: no field of those planes
+// has been formed, and they are then the noisy ones.
 void Domain::add_noise(float amplitude, uint64_t seed) {
+  if (!planes_given_) ensure_device_fields();
   form_planes();
   const int slot = state_slot();
   check(launch_init_planes(lattice_, storage_, d_sout_, amplitude, seed, buf_[slot], stride_, d_prev_, nx_,

@@ -251,7 +251,7 @@ class Domain {
   }
   void invalidate_mirrors() {
     drop_fields();
-    fsrc_valid_ = fdst_valid_ = sout_is_fsrc_ = false;
+    fsrc_valid_ = fdst_valid_ = sout_is_fsrc_ = planes_given_ = false;
   }
   void ensure_device_fields();
   void* alloc(size_t bytes);
@@ -405,6 +405,7 @@ class Domain {
   bool fsrc_valid_ = false, fdst_valid_ = false;
   bool sout_is_fsrc_ = false;  // d_sout_ holds the bytes of the current f_src() mirror
   bool dfields_valid_ = false;  // device moment arrays current
+  bool planes_given_ = false;   // FP32 planes were set and no step taken since
 };
 
 // splitmix64 finaliser (same constants as the device inlet turbulence).
