@@ -231,3 +231,18 @@ def test_fields_after_noise(wa, lattice, shape, storage):
         h.set_populations(g.f_src_data().copy())
         want = read(h)
     assert all(np.array_equal(a, b) for a, b in zip(read(g), want))
+
+
+@pytest.mark.parametrize("storage", [0, 1, 2])
+@pytest.mark.parametrize("lattice,shape", CASES)
+def test_setting_populations_takes_no_device_memory(wa, lattice, shape, storage):
+    """A domain admitted by its size can take its state: no scratch is kept."""
+    g = _grid(wa, lattice, shape, storage)
+    before = g.device_bytes()
+    f = np.random.default_rng(1).uniform(0.01, 0.4, (lattice, g.total_nodes())).astype(np.float32)
+    g.run(2, "BGK")
+    g.set_populations(f)
+    assert g.device_bytes() == before
+    one = _grid(wa, lattice, (8, 4, 2), 0)
+    one.initialize(1.0)
+    assert np.array_equal(g.f_src_data(), _stored(f, one.f_src_data()[:, 0].copy(), storage))

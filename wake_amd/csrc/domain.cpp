@@ -288,18 +288,26 @@ void Domain::initialize_fields(const float* rho, const float* ux, const float* u
   refresh_held();
 }
 
+// The planes go up through the moment arrays, five at a time: they hold
+// nothing after this, and a scratch of Q planes would double what a domain
+// with 16-bit storage takes.
 void Domain::set_populations(const float* f_ref) {
   before_config_change();
   const int slot = state_slot();
-  check(hipMemcpyAsync(planes_scratch(), f_ref, static_cast<size_t>(Q_) * N_ * sizeof(float), hipMemcpyHostToDevice,
-                       stream_),
-        "upload");
-  check(launch_init_planes(lattice_, storage_, d_sout_, 0.0f, 0, buf_[slot], stride_, d_prev_, nx_,
-                           static_cast<int>(N_), stream_),
-        "set populations");
+  invalidate_mirrors();
+  float* const stage[5] = {d_rho_, d_ux_, d_uy_, d_uz_, d_speed_};
+  for (int q = 0; q < Q_; q += 5) {
+    const int count = std::min(5, Q_ - q);
+    for (int k = 0; k < count; ++k)
+      check(hipMemcpyAsync(stage[k], f_ref + static_cast<size_t>(q + k) * N_, N_ * sizeof(float),
+                           hipMemcpyHostToDevice, stream_),
+            "upload");
+    check(launch_init_planes(lattice_, storage_, stage, q, count, 0.0f, 0, buf_[slot], stride_, d_prev_, nx_,
+                             static_cast<int>(N_), stream_),
+          "set populations");
+  }
   state_set(slot);
   check(hipStreamSynchronize(stream_), "upload");
-  invalidate_mirrors();
   planes_given_ = storage_ == kStoreF32;
   refresh_held();
 }
@@ -312,7 +320,9 @@ void Domain::add_noise(float amplitude, uint64_t seed) {
   if (!planes_given_) ensure_device_fields();
   form_planes();
   const int slot = state_slot();
-  check(launch_init_planes(lattice_, storage_, d_sout_, amplitude, seed, buf_[slot], stride_, d_prev_, nx_,
+  const float* planes[27];
+  for (int q = 0; q < Q_; ++q) planes[q] = d_sout_ + static_cast<size_t>(q) * N_;
+  check(launch_init_planes(lattice_, storage_, planes, 0, Q_, amplitude, seed, buf_[slot], stride_, d_prev_, nx_,
                            static_cast<int>(N_), stream_),
         "noise");
   state_set(slot);

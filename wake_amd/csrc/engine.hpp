@@ -181,11 +181,12 @@ hipError_t launch_readback_thermal(int storage, bool from_s, const StepArgs& a, 
 hipError_t launch_init_fields(int lattice, int storage, const float* rho, const float* ux, const float* uy,
                               const float* uz, float* speed, void* buf, long long stride, float* prev, int nx, int N,
                               hipStream_t s);
-// State from FP32 planes of N values, plus seeded noise U(-a, a) of counter
-// node * Q + q when amplitude is not zero.
-hipError_t launch_init_planes(int lattice, int storage, const float* planes, float amplitude,
-                              unsigned long long seed, void* buf, long long stride, float* prev, int nx, int N,
-                              hipStream_t s);
+// Populations q0 .. q0 + count - 1 of a state from as many FP32 planes of N
+// values, plus seeded noise U(-a, a) of counter node * Q + q when amplitude is
+// not zero.
+hipError_t launch_init_planes(int lattice, int storage, const float* const* planes, int q0, int count,
+                              float amplitude, unsigned long long seed, void* buf, long long stride, float* prev,
+                              int nx, int N, hipStream_t s);
 // Materialise S_k (commit=true updates the convective outlet store) into
 // s_state (storage format, stride a.stride), or fields/planes for read-back.
 hipError_t launch_materialize(int lattice, int storage, const StepArgs& a, const void* a_in, void* s_state,

@@ -69,17 +69,22 @@ __device__ __forceinline__ unsigned long long mix64(unsigned long long x) {
   return x ^ (x >> 31);
 }
 
-// FP32 planes (stride N) plus seeded noise (amplitude 0: none, the planes as
-// they are) -> the state.
+struct Planes {
+  const float* p[D3Q27::Q];
+};
+
+// FP32 planes of the populations q0 .. q1 - 1 plus seeded noise (amplitude 0:
+// none, the planes as they are) -> the state.
 template <class L, int STORAGE>
-__global__ __launch_bounds__(256) void k_init_planes(const float* __restrict__ planes, float amplitude,
+__global__ __launch_bounds__(256) void k_init_planes(const Planes planes, int q0, int q1, float amplitude,
                                                      unsigned long long seed, void* __restrict__ buf,
                                                      long long stride, float* __restrict__ prev, int nx, int N) {
   const int n = blockIdx.x * 256 + threadIdx.x;
   if (n >= N) return;
   static_for<L::Q>([&](auto qc) {
     constexpr int q = decltype(qc)::value;
-    float f = planes[static_cast<long long>(q) * N + n];
+    if (q < q0 || q >= q1) return;
+    float f = planes.p[q][n];
     if (amplitude != 0.0f) {
       const unsigned long long h = mix64(seed ^ (static_cast<unsigned long long>(n) * L::Q + q));
       const double u = static_cast<double>(h >> 40) * (1.0 / 16777216.0);
@@ -116,12 +121,15 @@ hipError_t launch_init_fields(int lattice, int storage, const float* rho, const 
   });
 }
 
-hipError_t launch_init_planes(int lattice, int storage, const float* planes, float amplitude,
-                              unsigned long long seed, void* buf, long long stride, float* prev, int nx, int N,
-                              hipStream_t s) {
+hipError_t launch_init_planes(int lattice, int storage, const float* const* planes, int q0, int count,
+                              float amplitude, unsigned long long seed, void* buf, long long stride, float* prev,
+                              int nx, int N, hipStream_t s) {
+  if (q0 < 0 || count < 0 || q0 + count > lattice) return hipErrorInvalidValue;
   return with_kind(lattice, storage, [&](auto lat, auto st) {
+    Planes p{};
+    for (int k = 0; k < count; ++k) p.p[q0 + k] = planes[k];
     k_init_planes<decltype(lat), decltype(st)::value>
-        <<<(N + 255) / 256, 256, 0, s>>>(planes, amplitude, seed, buf, stride, prev, nx, N);
+        <<<(N + 255) / 256, 256, 0, s>>>(p, q0, q0 + count, amplitude, seed, buf, stride, prev, nx, N);
     return hipGetLastError();
   });
 }
