@@ -327,6 +327,7 @@ class Domain {
   bool tile_kind() const;        // 2D without curved links or convective outlet, not switched off
   bool tile_eligible() const;
   bool plain_periodic() const;   // no node carries a class bit
+  bool moving_cells_ = false;    // a cell was set to MovingWall since the last initialize()
   bool all_fluid_ = false;       // every cell type Fluid (set with the class bytes)
   void step_tile(int nsteps, int collision, float gx, float gy, bool use_les, float smag);
   bool tile_enabled_ = true;     // run() may take up to kTbSteps steps per launch
