@@ -182,7 +182,10 @@ def _same_as_single_steps(wa, make, nx, ny, storage, coll, les=False, gx=0.0, gy
         g = make(wa, nx, ny, storage)
         g.set_multistep(multi)
         if probe:
+            # the node lists are built, then the history and the state set anew
             g.set_force_probe(nx / 3.0, ny / 2.0, 0.0, 0.0)
+            g.run(24, coll, gx=gx, gy=gy, use_les=les, smag=0.17)
+            g.add_noise(1e-4, 3)
         for steps in runs:
             g.run(steps, coll, gx=gx, gy=gy, use_les=les, smag=0.17)
         end = _state(g, thermal) + [g.f_dst_data().copy()]
@@ -256,5 +259,28 @@ def test_force_history_around_batch_steps(wa, gap, read):
         g.run(9, "MRT", use_les=True, smag=0.17)
         hist.append((f, g.force_history()[1]))
         assert len(hist[-1][1]) == 10
+    for a, b in zip(*hist):
+        assert np.array_equal(a, b)
+
+
+def test_force_history_of_short_runs(wa):
+    """Runs too short to pay for the node lists, geometries and probes that
+    change between them, and runs after the lists were built."""
+    hist = []
+    for multi in (True, False):
+        g = _channel(wa, 150, 50, 0)
+        g.set_multistep(multi)
+        g.set_force_probe(50.0, 25.0, 0.0, 20.0)
+        out = []
+        for k, steps in enumerate((7, 8, 8, 7, 9, 2, 40, 3, 8, 30, 1, 25)):
+            if k in (3, 7):
+                g.set_solid_box(90 + k, 20, 91 + k, 24)
+            if k == 9:
+                out.append(g.force_history()[1].copy())
+                g.set_force_probe(60.0, 25.0, 0.0, 30.0)
+            g.run(steps, "MRT", use_les=True, smag=0.17)
+        out.append(g.force_history()[1].copy())
+        assert [len(f) for f in out] == [93, 57]
+        hist.append(out)
     for a, b in zip(*hist):
         assert np.array_equal(a, b)

@@ -909,7 +909,7 @@ float Domain::run(int steps, int collision, float gx, float gy, float gz, bool u
     int s = 0;
     // 2D domains: up to kTbSteps steps per launch (an untimed run only: the
     // kernel timer samples single-step launches)
-    if (!timed && tile_eligible()) {
+    if (!timed && steps >= 2 && tile_eligible() && probe_lists(steps)) {
       const int most = tile2d_steps_of(nx_, ny_, thermal_ && storage_ == kStoreF32);
       while (steps - s >= 2) {
         const int k = std::min(steps - s, most);
@@ -1201,18 +1201,27 @@ int* Domain::build_mem_nodes(const MemRows& rows, float ccx, float ccy, float cc
   a.mem_c[2] = ccz;
   a.mem_rmax = r_max;
   int* d_cnt = static_cast<int*>(alloc(2 * static_cast<size_t>(nr) * sizeof(int)));
-  check(launch_mem_row_nodes(lattice_, a, rows.d_list, nr, d_cnt, nullptr, nullptr, stream_), "link nodes");
-  std::vector<int> cnt(nr), off(nr);
-  check(hipMemcpyAsync(cnt.data(), d_cnt, nr * sizeof(int), hipMemcpyDeviceToHost, stream_), "link nodes");
-  check(hipStreamSynchronize(stream_), "link nodes");
-  for (int r = 0; r < nr; ++r) {
-    off[r] = *count;
-    *count += cnt[r];
+  int* d_nodes = nullptr;
+  try {
+    check(launch_mem_row_nodes(lattice_, a, rows.d_list, nr, d_cnt, nullptr, nullptr, stream_), "link nodes");
+    std::vector<int> cnt(nr), off(nr);
+    check(hipMemcpyAsync(cnt.data(), d_cnt, nr * sizeof(int), hipMemcpyDeviceToHost, stream_), "link nodes");
+    check(hipStreamSynchronize(stream_), "link nodes");
+    for (int r = 0; r < nr; ++r) {
+      off[r] = *count;
+      *count += cnt[r];
+    }
+    d_nodes = static_cast<int*>(alloc(std::max(1, *count) * sizeof(int)));
+    check(hipMemcpyAsync(d_cnt + nr, off.data(), nr * sizeof(int), hipMemcpyHostToDevice, stream_), "link nodes");
+    check(launch_mem_row_nodes(lattice_, a, rows.d_list, nr, d_cnt, d_cnt + nr, d_nodes, stream_), "link nodes");
+    check(hipStreamSynchronize(stream_), "link nodes");
+  } catch (...) {
+    (void)hipStreamSynchronize(stream_);
+    release(d_nodes);
+    release(d_cnt);
+    *count = 0;
+    throw;
   }
-  int* d_nodes = static_cast<int*>(alloc(std::max(1, *count) * sizeof(int)));
-  check(hipMemcpyAsync(d_cnt + nr, off.data(), nr * sizeof(int), hipMemcpyHostToDevice, stream_), "link nodes");
-  check(launch_mem_row_nodes(lattice_, a, rows.d_list, nr, d_cnt, d_cnt + nr, d_nodes, stream_), "link nodes");
-  check(hipStreamSynchronize(stream_), "link nodes");
   release(d_cnt);
   return d_nodes;
 }
@@ -1303,7 +1312,7 @@ void Domain::set_force_probe(float ccx, float ccy, float ccz, float r_max) {
   // geometry (probe_epoch_): a restart of the same probe keeps them
   if (!probe_ || probe_c_[0] != ccx || probe_c_[1] != ccy || probe_c_[2] != ccz || probe_rmax_ != r_max) {
     if (probe_rows_.d_rows) free_mem_rows(probe_rows_);
-    probe_epoch_ = tile_epoch_ = ~0ull;
+    probe_epoch_ = tile_epoch_ = wait_epoch_ = ~0ull;
   }
   probe_ = true;
   probe_c_[0] = ccx;
@@ -1375,6 +1384,46 @@ double* Domain::probe_slot(uint64_t k) {
   return d_ring_ + 3 * static_cast<size_t>(std::max(1, probe_rows_.nslots)) * (k % kForceRing);
 }
 
+// Whether the next `steps` steps may leave their samples through tile
+// launches: the list of the nodes holding links, and the sums of a ring of
+// steps for each.
+bool Domain::probe_lists(int steps) {
+  if (!probe_ || fh_next_ < step_count_) return true;  // no samples are taken
+  probe_sync();
+  if (tile_epoch_ == probe_epoch_) return tile_lists_;
+  // Building them takes 60 us (240 x 80) to 90 us (1500 x 403 nodes), a tile
+  // launch saves 3.6 to 4.6 us a step: they pay after 17 to 20 steps.  Until
+  // then a geometry or a probe that changes from run to run takes single steps.
+  if (wait_epoch_ != probe_epoch_) wait_steps_ = 0;
+  wait_epoch_ = probe_epoch_;
+  if (steps < kListSteps - wait_steps_) {
+    wait_steps_ += steps;
+    return false;
+  }
+  if (d_findex_ || d_fnode_) check(hipStreamSynchronize(stream_), "force nodes");
+  free_tile_lists();
+  int* d_nodes = build_mem_nodes(probe_rows_, probe_c_[0], probe_c_[1], probe_c_[2], probe_rmax_, &n_fnodes_);
+  if (n_fnodes_ > 0) {
+    d_findex_ = static_cast<int*>(alloc(N_ * sizeof(int)));
+    d_fnode_ = static_cast<double*>(alloc(3 * sizeof(double) * kForceRing * static_cast<size_t>(n_fnodes_)));
+    check(hipMemsetAsync(d_findex_, 0xff, N_ * sizeof(int), stream_), "force nodes");
+    check(launch_index_nodes(d_nodes, n_fnodes_, d_findex_, stream_), "force nodes");
+    check(hipStreamSynchronize(stream_), "force nodes");
+  }
+  release(d_nodes);
+  tile_lists_ = true;
+  tile_epoch_ = probe_epoch_;
+  return true;
+}
+
+void Domain::free_tile_lists() {
+  release(d_findex_);
+  release(d_fnode_);
+  d_findex_ = nullptr;
+  d_fnode_ = nullptr;
+  n_fnodes_ = 0;
+}
+
 // Samples a tile launch of nsteps steps from step_count_ takes: S_{fh_next_}
 // up to S_{step_count_ + nsteps - 1}, as per-node sums in d_fnode_ until
 // probe_flush_tiles() turns them into the ring's partials.
@@ -1384,24 +1433,6 @@ TileForces Domain::probe_tile(int nsteps) {
     tile_first_ = tile_end_ = fh_next_;
   }
   if (step_count_ + nsteps - fh_folded_ > static_cast<uint64_t>(kForceRing)) probe_fold(fh_next_);
-  if (tile_epoch_ != probe_epoch_) {
-    if (d_findex_ || d_fnode_) check(hipStreamSynchronize(stream_), "force nodes");
-    release(d_findex_);
-    release(d_fnode_);
-    d_findex_ = nullptr;
-    d_fnode_ = nullptr;
-    int* d_nodes =
-        build_mem_nodes(probe_rows_, probe_c_[0], probe_c_[1], probe_c_[2], probe_rmax_, &n_fnodes_);
-    if (n_fnodes_ > 0) {
-      d_findex_ = static_cast<int*>(alloc(N_ * sizeof(int)));
-      d_fnode_ = static_cast<double*>(alloc(3 * sizeof(double) * kForceRing * static_cast<size_t>(n_fnodes_)));
-      check(hipMemsetAsync(d_findex_, 0xff, N_ * sizeof(int), stream_), "force nodes");
-      check(launch_index_nodes(d_nodes, n_fnodes_, d_findex_, stream_), "force nodes");
-      check(hipStreamSynchronize(stream_), "force nodes");
-    }
-    release(d_nodes);
-    tile_epoch_ = probe_epoch_;
-  }
   return TileForces{d_findex_, d_fnode_, n_fnodes_, kForceRing};
 }
 

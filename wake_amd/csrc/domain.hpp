@@ -279,6 +279,8 @@ class Domain {
   void probe_sample_current();      // sample S_{step_count_} if no launch has
   double* probe_slot(uint64_t k);   // ring entry of step k (folding first if it is taken)
   TileForces probe_tile(int nsteps);  // where the next tile launch writes its samples
+  bool probe_lists(int steps);        // what tile launches need to take the samples of `steps` steps
+  void free_tile_lists();
   void probe_flush_tiles();         // partials of the samples tile launches left
   void probe_restart();
 
@@ -373,6 +375,10 @@ class Domain {
   double* d_fnode_ = nullptr;
   int n_fnodes_ = 0;
   uint64_t tile_first_ = 0, tile_end_ = 0;
+  bool tile_lists_ = false;  // they are there for tile_epoch_ (or not needed: no links)
+  static constexpr int kListSteps = 24;
+  uint64_t wait_epoch_ = ~0ull;  // steps taken without them at this epoch
+  int wait_steps_ = 0;
   double* d_ring_ = nullptr;
   size_t ring_cap_ = 0;  // in doubles
   double* d_fhist_ = nullptr;
