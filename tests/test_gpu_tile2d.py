@@ -263,6 +263,15 @@ def test_force_history_around_batch_steps(wa, gap, read):
         assert np.array_equal(a, b)
 
 
+def _porous(wa, nx, ny, storage):
+    g = _channel(wa, nx, ny, storage)
+    x, y = np.meshgrid(np.arange(nx), np.arange(ny))
+    for i, j in zip(x[(x + y) % 3 == 0], y[(x + y) % 3 == 0]):
+        if 4 < i < nx - 4:
+            g.set_cell_type(int(i), int(j), 1)
+    return g
+
+
 def test_force_history_of_short_runs(wa):
     """Runs too short to pay for the node lists, geometries and probes that
     change between them, and runs after the lists were built."""
@@ -284,3 +293,21 @@ def test_force_history_of_short_runs(wa):
         hist.append(out)
     for a, b in zip(*hist):
         assert np.array_equal(a, b)
+
+
+def test_force_samples_of_a_porous_body(wa):
+    """The lists of a tile launch's samples are bounded by the state's size:
+    a body with a link in most nodes is sampled by single steps."""
+    nx, ny = 512, 300
+    hist = []
+    for multi in (True, False):
+        g = _porous(wa, nx, ny, 0)
+        g.set_multistep(multi)
+        g.run(2, "TRT")
+        before = g.device_bytes()
+        g.set_force_probe(nx / 2.0, ny / 2.0, 0.0, 0.0)
+        g.run(3, "TRT")
+        g.run(60, "TRT")
+        assert g.device_bytes() - before < 64 << 20
+        hist.append(g.force_history()[1])
+    assert np.array_equal(*hist)

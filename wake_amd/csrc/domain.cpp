@@ -1402,18 +1402,27 @@ bool Domain::probe_lists(int steps) {
   }
   if (d_findex_ || d_fnode_) check(hipStreamSynchronize(stream_), "force nodes");
   free_tile_lists();
-  int* d_nodes = build_mem_nodes(probe_rows_, probe_c_[0], probe_c_[1], probe_c_[2], probe_rmax_, &n_fnodes_);
-  if (n_fnodes_ > 0) {
-    d_findex_ = static_cast<int*>(alloc(N_ * sizeof(int)));
-    d_fnode_ = static_cast<double*>(alloc(3 * sizeof(double) * kForceRing * static_cast<size_t>(n_fnodes_)));
-    check(hipMemsetAsync(d_findex_, 0xff, N_ * sizeof(int), stream_), "force nodes");
-    check(launch_index_nodes(d_nodes, n_fnodes_, d_findex_, stream_), "force nodes");
-    check(hipStreamSynchronize(stream_), "force nodes");
+  tile_epoch_ = probe_epoch_;
+  int* d_nodes = nullptr;
+  try {
+    d_nodes = build_mem_nodes(probe_rows_, probe_c_[0], probe_c_[1], probe_c_[2], probe_rmax_, &n_fnodes_);
+    // (a porous body can hold a link in every other node: past the size of
+    // the state itself its samples are left to single steps)
+    const size_t sums = 3 * sizeof(double) * kForceRing * static_cast<size_t>(n_fnodes_);
+    tile_lists_ = sums <= std::max<size_t>(64u << 20, 2 * static_cast<size_t>(Q_) * stride_ * elem_);
+    if (tile_lists_ && n_fnodes_ > 0) {
+      d_findex_ = static_cast<int*>(alloc(N_ * sizeof(int)));
+      d_fnode_ = static_cast<double*>(alloc(sums));
+      check(hipMemsetAsync(d_findex_, 0xff, N_ * sizeof(int), stream_), "force nodes");
+      check(launch_index_nodes(d_nodes, n_fnodes_, d_findex_, stream_), "force nodes");
+      check(hipStreamSynchronize(stream_), "force nodes");
+    }
+  } catch (const HipError&) {
+    tile_lists_ = false;  // no memory for them: single steps take the samples
   }
   release(d_nodes);
-  tile_lists_ = true;
-  tile_epoch_ = probe_epoch_;
-  return true;
+  if (!tile_lists_) free_tile_lists();
+  return tile_lists_;
 }
 
 void Domain::free_tile_lists() {
