@@ -333,6 +333,17 @@ class Batch {
     const int n = static_cast<int>(members_.size());
     if (!shape_explicit_) shape_.block = default_block();
     span_ = pick_span();
+    // where there is no memory for the tiles' force sums, single steps take them
+    try {
+      for (const Member& m : members_) {
+        if (span_ == 1 || !m.forces) continue;
+        int count = 0;
+        (void)m.d->batch_mem_nodes(m.c[0], m.c[1], m.c[2], m.r_max, &count);
+        (void)m.d->batch_tile_forces();
+      }
+    } catch (const HipError&) {
+      span_ = 1;
+    }
     any_g_ = false;
     std::vector<BatchSlot> slots(n);
     std::vector<int> tile_slot;

@@ -1584,8 +1584,9 @@ const int* Domain::batch_mem_nodes(float ccx, float ccy, float ccz, float r_max,
     d_batch_index_ = nullptr;
     d_batch_sums_ = nullptr;
     batch_rows_ = build_mem_rows(ccx, ccy, ccz, r_max);
-    batch_rows_key_ = key;
+    batch_rows_key_ = {0.0f, 0.0f, 0.0f, 0.0f, ~0ull};  // (none, should the next line throw)
     d_batch_nodes_ = build_mem_nodes(batch_rows_, ccx, ccy, ccz, r_max, &n_batch_nodes_);
+    batch_rows_key_ = key;
   }
   *count = n_batch_nodes_;
   return d_batch_nodes_;
@@ -1593,11 +1594,21 @@ const int* Domain::batch_mem_nodes(float ccx, float ccy, float ccz, float r_max,
 
 TileForces Domain::batch_tile_forces() {
   if (n_batch_nodes_ > 0 && !d_batch_index_) {
-    d_batch_index_ = static_cast<int*>(alloc(N_ * sizeof(int)));
-    d_batch_sums_ = static_cast<double*>(alloc(3 * sizeof(double) * kTbSteps * static_cast<size_t>(n_batch_nodes_)));
-    check(hipMemsetAsync(d_batch_index_, 0xff, N_ * sizeof(int), stream_), "batch nodes");
-    check(launch_index_nodes(d_batch_nodes_, n_batch_nodes_, d_batch_index_, stream_), "batch nodes");
-    check(hipStreamSynchronize(stream_), "batch nodes");  // the batch runs on its own stream
+    int* index = static_cast<int*>(alloc(N_ * sizeof(int)));
+    double* sums = nullptr;
+    try {
+      sums = static_cast<double*>(alloc(3 * sizeof(double) * kTbSteps * static_cast<size_t>(n_batch_nodes_)));
+      check(hipMemsetAsync(index, 0xff, N_ * sizeof(int), stream_), "batch nodes");
+      check(launch_index_nodes(d_batch_nodes_, n_batch_nodes_, index, stream_), "batch nodes");
+      check(hipStreamSynchronize(stream_), "batch nodes");  // the batch runs on its own stream
+    } catch (...) {
+      (void)hipStreamSynchronize(stream_);
+      release(sums);
+      release(index);
+      throw;
+    }
+    d_batch_index_ = index;  // both or neither: the tiles write the sums of every indexed node
+    d_batch_sums_ = sums;
   }
   return TileForces{d_batch_index_, d_batch_sums_, n_batch_nodes_, kTbSteps};
 }
