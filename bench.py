@@ -13,8 +13,8 @@ By default the line also nests the metric's batched-serve half: a
 against its plain one-at-a-time path (`--sub-records none` skips them).
 
 `--workload batched-wakes` runs the batched multi-domain path alone: 512
-D2Q9 MRT cylinder-wake domains of uneven size, one launch per step over all
-of them, and compares simulations per second with the plain
+D2Q9 MRT cylinder-wake domains of uneven size, stepped together (up to 8
+steps per launch over all of them), and compares simulations per second with the plain
 one-domain-at-a-time path.  `--workload serve` replays a Poisson stream of
 mixed 3D bluff-body and 2D thermal-cavity requests through the
 continuous-batching serving loop and then through the plain sequential
@@ -184,9 +184,10 @@ def batched_wakes(wa, ndom, seed=4, umax=0.05, storage=0):
 
 
 def batched_record(args):
-    """Batched cylinder wakes: every domain stepped `steps` times by one
-    launch per step (graph-captured chunks of 100, autotuned launch shape),
-    force history per step, C_D and Strouhal per domain; the plain
+    """Batched cylinder wakes: every domain stepped `steps` times by launches
+    over all of them (several steps each where the domains allow it, else one
+    with an autotuned shape; graph-captured chunks of 100), force history per
+    step, C_D and Strouhal per domain; the plain
     one-domain-at-a-time path (the single-domain step with the same per-step
     force, taken inside its step launch) is timed per domain on a short run
     and scaled to the same step count.  Returns the record as a dict."""
@@ -226,7 +227,8 @@ def batched_record(args):
     shape = b.tune(probe_steps=4)
     tune_s = time.perf_counter() - t0
     left = max(b.remaining(s) for s in slots)
-    log(f"autotuned launch shape block={shape[0]} grid_factor={shape[1]} in {tune_s:.2f}s; {left} steps left")
+    log(f"single-step launch shape block={shape[0]} grid_factor={shape[1]} ({tune_s:.2f}s tuning; no effect on "
+        f"launches of several steps); {left} steps left")
     t0 = time.perf_counter()
     ms = b.run(left, use_graph=not getattr(args, "no_graph", False))
     wall = time.perf_counter() - t0
@@ -263,7 +265,7 @@ def batched_record(args):
         "config": {
             "workload": f"{ndom} D2Q9 MRT+Smagorinsky(Cs=0.17) cylinder wakes (NX 128-1024 step 32, NY=NX/4, D=NY/8, "
                         f"parabolic Zou-He inlet umax=0.05, Re 50-300 log-uniform, seed 4), {S} steps each with the "
-                        f"force of every step, one launch per step over all domains, graph chunks of 100 steps",
+                        f"force of every step, stepped together, graph chunks of 100 steps",
             "nodes": nodes, "launch_shape": {"block": shape[0], "grid_factor": shape[1]},
             "batched_mlups": round(mlups, 1), "plain_sims_per_s": round(ndom / t_plain, 4),
             "batched_gbps": round(gbps, 1), "pull_d2q9_gbps": round(pull9, 1),

@@ -405,12 +405,14 @@ int wake_thermal2d_stats(wake_thermal2d* t, double out[2]);
  * reference, which steps one grid per call of LatticeGrid*::step,
  * src/grid/lattice_grid_2d.cpp:195-265 and lattice_grid_3d.cpp:301-380).
  *
- * A batch steps every member domain with one kernel launch per step.  The
- * members share lattice, population storage, collision and LES coupling and
+ * A batch steps every member domain with one kernel launch per step, or per
+ * 4 or 8 steps where every member is a 2D domain that wake_domain_run would
+ * take several steps per launch of (wake_domain_set_multistep).  The members
+ * share lattice, population storage, collision and LES coupling and
  * keep everything else of their own (size, cell types, boundaries, tau,
  * body force).  Each member takes exactly the steps it was added with; a
  * member's results are those of stepping it alone.  Steps run in chunks of
- * `chunk` launches captured once as a HIP graph.  A domain must not be
+ * `chunk` steps captured once as a HIP graph.  A domain must not be
  * stepped, destroyed or added to another batch while it is a member; after
  * wake_batch_run returns its fields and populations read as after
  * wake_domain_step.
@@ -429,10 +431,10 @@ void wake_batch_destroy(wake_batch* b);
 int wake_batch_add(wake_batch* b, wake_domain* d, long long steps, float gx, float gy, float gz, float smag,
                    int track_forces, float cx, float cy, float cz, float r_max, int* slot);
 int wake_batch_remove(wake_batch* b, int slot);
-/* `steps` launches (each member takes min(steps, its remaining steps));
- * *ms = device time.  use_graph = 0 launches each step directly. */
+/* `steps` steps (each member takes min(steps, its remaining steps));
+ * *ms = device time.  use_graph = 0 launches without a graph. */
 int wake_batch_run(wake_batch* b, long long steps, int use_graph, float* ms);
-/* Asynchronous form: enqueue one chunk (min(steps, chunk) launches) on the
+/* Asynchronous form: enqueue one chunk (min(steps, chunk) steps) on the
  * batch's own stream and return; wake_batch_wait completes it (*ms = device
  * time).  Chunks of different batches in flight together overlap on the
  * GPU.  No other call on the batch or its members until the wait. */
@@ -445,7 +447,8 @@ int wake_batch_forces(wake_batch* b, int slot, double* out, long long capacity, 
 /* Autotuner: times probe_steps real steps under each candidate launch shape
  * (work-group size; one work-group per tile or a persistent grid of
  * grid_factor x compute units) and keeps the fastest.  The steps count as
- * steps of the members. */
+ * steps of the members.  Launches of several 2D steps have one shape: there
+ * no step is taken and the shape in force is returned. */
 int wake_batch_tune(wake_batch* b, int probe_steps, int* block, int* grid_factor);
 /* Fix the launch shape.  Until this or wake_batch_tune is called, the
  * work-group width is the one of 256 / 128 / 64 that leaves the fewest idle

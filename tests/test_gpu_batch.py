@@ -127,6 +127,31 @@ def test_batch_tune_and_graph_do_not_change_results(wa):
         assert np.array_equal(x.f_src_data(), y.f_src_data())
 
 
+def test_batch_tune_times_single_step_launches_only(wa):
+    """Where the members take several steps per launch the shape has no effect:
+    tuning takes no step and leaves the shapes of single-step batches alone."""
+    ends = []
+    for multi in (True, False):
+        b = wa.Batch(lattice=9, collision="TRT", chunk=8)
+        grids = [cylinder_channel(wa, nx, off)[0] for nx, off in SIZES]
+        for g in grids:
+            g.set_multistep(multi)
+        slots = [b.add(g, 60) for g in grids]
+        before = b.info()
+        shape = b.tune(probe_steps=2)
+        left = [b.remaining(s) for s in slots]
+        assert shape[0] in (64, 128, 256)
+        if multi:
+            assert left == [60] * len(slots) and (before["block"], before["grid_factor"]) == shape
+        else:
+            # (a winner left by the tile launches above would be taken without a step)
+            assert max(left) < 60
+        b.run(60)
+        ends.append([g.f_src_data().copy() for g in grids])
+    for x, y in zip(*ends):
+        assert np.array_equal(x, y)
+
+
 def test_batch_membership_changes_and_mixed_progress(wa):
     batch = wa.Batch(lattice=9, collision="MRT", chunk=10)
     g0, _ = cylinder_channel(wa, 128, 0)

@@ -50,14 +50,14 @@ class Batch:
         self._members.pop(slot, None)
 
     def run(self, steps, use_graph=True):
-        """Run `steps` launches; returns the device time in ms."""
+        """Run `steps` steps; returns the device time in ms."""
         ms = ctypes.c_float()
         _lib.check(self._L.wake_batch_run(self._h, int(steps), int(bool(use_graph)), ctypes.byref(ms)),
                    "wake_batch_run")
         return ms.value
 
     def launch(self, steps, use_graph=True):
-        """Enqueue one chunk (min(steps, chunk) launches) and return at once."""
+        """Enqueue one chunk (min(steps, chunk) steps) and return at once."""
         _lib.check(self._L.wake_batch_launch(self._h, int(steps), int(bool(use_graph))), "wake_batch_launch")
 
     def wait(self):
@@ -81,7 +81,8 @@ class Batch:
         return out
 
     def tune(self, probe_steps=4):
-        """Autotune the launch shape on real steps; returns (block, grid_factor)."""
+        """Autotune the launch shape on real steps; returns (block, grid_factor).
+        Launches of several 2D steps have one shape: no step is taken there."""
         b, gf = ctypes.c_int(), ctypes.c_int()
         _lib.check(self._L.wake_batch_tune(self._h, int(probe_steps), ctypes.byref(b), ctypes.byref(gf)),
                    "wake_batch_tune")

@@ -1,14 +1,15 @@
 // batch_host.cpp -- host side of the batched multi-domain step, and its C ABI.
 //
-// A Batch steps many Domains of one lattice / storage / collision kind with
-// one kernel launch per step.  Steps run in chunks of `chunk` launches; a
-// full chunk is captured once as a HIP graph (step launches, per-step force
-// reductions, the slot-advance kernel) and replayed while the membership and
-// launch shape stay the same.  Each slot carries its own stop step, so every
-// domain takes exactly the steps it asked for even when a chunk would pass
-// them.  The autotuner times real steps under each candidate launch shape;
-// results do not depend on the shape (a node's arithmetic is the same in any
-// tile), so tuning costs no accuracy, only the steps it spends.
+// A Batch steps many Domains of one lattice / storage / collision kind
+// together: one kernel launch per step, or per 4 or 8 steps where every
+// member may take 2D tile launches.  Steps run in chunks of `chunk`; a full
+// chunk is captured once as a HIP graph (step launches, force reductions, the
+// slot-advance kernel) and replayed while the membership and launch shape
+// stay the same.  Each slot carries its own stop step, so every domain takes
+// exactly the steps it asked for even when a chunk would pass them.  The
+// autotuner times real steps under each candidate shape of single-step
+// launches; results do not depend on the shape (a node's arithmetic is the
+// same in any tile), so tuning costs no accuracy, only the steps it spends.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -194,6 +195,9 @@ class Batch {
   LaunchShape tune(int probe) {
     if (pending_) throw HipError("a chunk of this batch is in flight: wait first");
     prepare();
+    // tile launches have one shape: there is nothing to time, and a winner by
+    // noise would be given to single-step batches of the same class
+    if (span_ > 1) return shape();
     // the row-length class (the width that wastes the fewest lanes on the
     // members' rows) is part of the key: a shape tuned for long rows is not
     // reused for a batch of short ones of similar total size

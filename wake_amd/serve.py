@@ -3,8 +3,8 @@
 Requests (3D bluff-body runs, 2D thermal cavities) arrive over time.  Each
 admitted request becomes a Domain whose populations stay in HBM until its
 last step; requests of one kind (lattice, population storage, collision,
-LES, temperature coupling) share a Batch that advances all of them with one
-launch per step.  At every chunk boundary the loop completes the chunks in
+LES, temperature coupling) share a Batch that advances all of them together.
+At every chunk boundary the loop completes the chunks in
 flight (one per batch, each on its own stream, so the kinds overlap on the
 GPU), retires the requests that reached their step count, puts in the
 domains built meanwhile and launches the next chunk; while that chunk runs
