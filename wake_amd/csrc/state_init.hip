@@ -95,6 +95,11 @@ __global__ __launch_bounds__(256) void k_init_planes(const Planes planes, int q0
   });
 }
 
+// (a domain may hold up to 2^31 - 1 nodes)
+constexpr unsigned blocks_of(int nodes) { return (static_cast<unsigned>(nodes) + 255u) / 256u; }
+static_assert(blocks_of(0x7fffffff) == 1u << 23 && blocks_of(0x7fffff01) == 1u << 23 &&
+              blocks_of(0x7fffff00) == (1u << 23) - 1 && blocks_of(257) == 2 && blocks_of(1) == 1);
+
 template <class F>
 hipError_t with_kind(int lattice, int storage, F&& f) {
   auto with = [&](auto lat) {
@@ -116,7 +121,7 @@ hipError_t launch_init_fields(int lattice, int storage, const float* rho, const 
                               hipStream_t s) {
   return with_kind(lattice, storage, [&](auto lat, auto st) {
     k_init_fields<decltype(lat), decltype(st)::value>
-        <<<(N + 255) / 256, 256, 0, s>>>(rho, ux, uy, uz, speed, buf, stride, prev, nx, N);
+        <<<blocks_of(N), 256, 0, s>>>(rho, ux, uy, uz, speed, buf, stride, prev, nx, N);
     return hipGetLastError();
   });
 }
@@ -129,7 +134,7 @@ hipError_t launch_init_planes(int lattice, int storage, const float* const* plan
     Planes p{};
     for (int k = 0; k < count; ++k) p.p[q0 + k] = planes[k];
     k_init_planes<decltype(lat), decltype(st)::value>
-        <<<(N + 255) / 256, 256, 0, s>>>(p, q0, q0 + count, amplitude, seed, buf, stride, prev, nx, N);
+        <<<blocks_of(N), 256, 0, s>>>(p, q0, q0 + count, amplitude, seed, buf, stride, prev, nx, N);
     return hipGetLastError();
   });
 }
