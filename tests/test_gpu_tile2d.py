@@ -311,3 +311,107 @@ def test_force_samples_of_a_porous_body(wa):
         assert g.device_bytes() - before < 64 << 20
         hist.append(g.force_history()[1])
     assert np.array_equal(*hist)
+
+
+# One size for each instance of the tile kernels besides the 32 x 24 tile of
+# the sizes above: 32 x 32 tiles of 8 steps (more than 256 low tiles, at most
+# 512 high ones; 256 with FP32 temperature), and of 4 steps beyond.
+EIGHT, FOUR = (259, 250), (530, 263)
+
+
+def _tiles(nx, ny, w, h):
+    return -(-nx // w) * -(-ny // h)
+
+
+def test_sizes_reach_their_instances():
+    assert _tiles(*EIGHT, 16, 8) > 256 and _tiles(*EIGHT, 16, 16) <= 512
+    assert _tiles(*FOUR, 16, 16) > 512
+    assert _tiles(240, 250, 16, 8) > 256 and _tiles(240, 250, 16, 16) <= 256
+    assert _tiles(*EIGHT, 16, 16) > 256  # FP32 temperature: 4 steps from here
+
+
+@pytest.mark.parametrize("force", [False, True])
+@pytest.mark.parametrize("storage", [0, 1, 2])
+@pytest.mark.parametrize("coll,les", [("BGK", False), ("BGK", True), ("TRT", False), ("TRT", True), ("MRT", False),
+                                      ("MRT", True)])
+@pytest.mark.parametrize("nx,ny", [EIGHT, FOUR])
+def test_larger_tiles_with_edges(wa, nx, ny, coll, les, storage, force):
+    gx, gy = (1e-6, -2e-6) if force else (0.0, 0.0)
+    _same_as_single_steps(wa, _thick_channel, nx, ny, storage, coll, les, gx, gy, probe=True, runs=(1, 3, 8, 13))
+    _same_as_single_steps(wa, _lid, nx, ny, storage, coll, False, gx, gy, runs=(5, 8))
+
+
+def _vortex(wa, nx, ny, storage):
+    g = wa.LatticeGrid2D(nx, ny, 0.7, storage=storage)
+    _start(g, nx, ny, 4)
+    g.set_les_coupled(True)
+    g.set_periodic(True)
+    return g
+
+
+@pytest.mark.parametrize("force", [False, True])
+@pytest.mark.parametrize("storage", [0, 1, 2])
+@pytest.mark.parametrize("coll,les", [("BGK", False), ("BGK", True), ("TRT", False), ("TRT", True), ("MRT", False),
+                                      ("MRT", True)])
+@pytest.mark.parametrize("nx,ny", [(240, 80), EIGHT, FOUR])
+def test_larger_tiles_of_periodic_domains(wa, nx, ny, coll, les, storage, force):
+    gx, gy = (1e-6, -2e-6) if force else (0.0, 0.0)
+    _same_as_single_steps(wa, _vortex, nx, ny, storage, coll, les, gx, gy, runs=(1, 3, 8, 13))
+
+
+@pytest.mark.parametrize("storage", [0, 1])
+@pytest.mark.parametrize("coll", ["BGK", "TRT", "MRT"])
+@pytest.mark.parametrize("nx,ny", [(240, 250), EIGHT, FOUR])
+def test_larger_tiles_with_temperature(wa, nx, ny, coll, storage):
+    _same_as_single_steps(wa, _warm_cavity, nx, ny, storage, coll, gx=1e-6, gy=-2e-6, thermal=True,
+                          runs=(1, 3, 8, 13))
+
+
+@pytest.mark.parametrize("force", [False, True])
+@pytest.mark.parametrize("storage", [0, 1, 2])
+@pytest.mark.parametrize("coll,les", [("BGK", False), ("BGK", True), ("TRT", False), ("TRT", True), ("MRT", False),
+                                      ("MRT", True)])
+@pytest.mark.parametrize("sizes", [[(96, 40), (33, 17)], [FOUR, (96, 40)]])
+def test_batch_tiles_of_both_spans(wa, sizes, coll, les, storage, force):
+    """Eight steps per launch, and four once the batch has more than 512 tiles."""
+    few = sum(_tiles(nx, ny, 16, 16) for nx, ny in sizes) <= 512
+    assert few == (sizes[0] != FOUR)
+    ends = []
+    for multi in (True, False):
+        grids = [_thick_channel(wa, nx, ny, storage) for nx, ny in sizes]
+        for g in grids:
+            g.set_les_coupled(les)
+            g.set_multistep(multi)
+        b = wa.Batch(lattice=9, storage=storage, collision=coll, use_les=les, chunk=11)
+        ids = [b.add(g, k, g=(1e-6, -1e-6, 0.0) if force else (0.0, 0.0, 0.0), smag=0.17,
+                     forces=(nx / 3.0, ny / 2.0, 0.0, 0.0))
+               for g, k, (nx, ny) in zip(grids, (23, 14), sizes)]
+        b.run(23)
+        end = [b.forces(i) for i in ids]
+        for g in grids:
+            end += _state(g, False) + [g.f_dst_data().copy()]
+        ends.append(end)
+    for a, c in zip(*ends):
+        assert np.array_equal(a, c, equal_nan=True)
+
+
+@pytest.mark.parametrize("storage", [0, 1])
+@pytest.mark.parametrize("coll", ["BGK", "TRT", "MRT"])
+@pytest.mark.parametrize("sizes", [[(96, 40), (33, 17)], [FOUR, (96, 40)]])
+def test_batch_tiles_of_cavities(wa, sizes, coll, storage):
+    """The members end as when stepped alone, one launch per step."""
+    ends = []
+    for batched in (True, False):
+        grids = [_warm_cavity(wa, nx, ny, storage) for nx, ny in sizes]
+        if batched:
+            b = wa.Batch(lattice=9, storage=storage, collision=coll, chunk=11, thermal=True)
+            for g, k in zip(grids, (23, 14)):
+                b.add(g, k)
+            b.run(23)
+        else:
+            for g, k in zip(grids, (23, 14)):
+                g.set_multistep(False)
+                g.run(k, coll)
+        ends.append([v for g in grids for v in _state(g, True)])
+    for a, c in zip(*ends):
+        assert np.array_equal(a, c, equal_nan=True)
