@@ -201,9 +201,15 @@ __device__ __forceinline__ void tile2d_steps(Tile2dShared<St, THERMAL, W, H>& sh
     }
     if (i >= s && i < W - s && j >= s && j < H - s) {
       float f[L::Q];
-      const bool formed = !(from_s && s == 1);  // S of this step is formed here, not given
-      const bool pull = formed && !(EDGE && (c & kClsFrozen));
+      const bool pull = !(from_s && s == 1) && !(EDGE && (c & kClsFrozen));
       const unsigned long long k = s_step + static_cast<unsigned long long>(s - 1);  // S_k is formed here
+      auto close = [&]() {
+        if (c & kClsInlet) {
+          if (noisy) u_edge = inlet_velocity(e, y, n, k);
+          close_inlet<L>(f, u_edge, e.uin_y);
+        }
+        if ((c & kClsOutlet) && e.outflow == 1) apply_zh_outflow_d2q9(e, f);
+      };
       static_for<L::Q>([&](auto qc) {
         constexpr int q = decltype(qc)::value;
         f[q] = tb_get<St, L, q>(sh.f[src][q][cell - L::cy[q] * W - L::cx[q]]);
@@ -213,41 +219,38 @@ __device__ __forceinline__ void tile2d_steps(Tile2dShared<St, THERMAL, W, H>& sh
           constexpr int q = decltype(qc)::value;
           f[q] = tb_get<St, L, q>(sh.f[src][q][cell]);
         });
-      } else if (EDGE && (c & kClsSlow)) {
-        // every own-node value is read at once and the bouncing ones kept:
-        // one LDS round trip instead of one per bouncing direction
-        float own_f[L::Q];
-        static_for<L::Q>([&](auto qc) {
-          constexpr int q = decltype(qc)::value;
-          if constexpr (q > 0) own_f[q] = tb_get<St, L, L::opp[q]>(sh.f[src][L::opp[q]][cell]);
-        });
-        if (moving) {
-          TileArgs* p = opaque_args(ap);
-          const float uw[3] = {p->uw[0], p->uw[1], p->uw[2]};
+        // solid nodes in the inlet and outlet rows are closed too, as form_s_at does
+        if (EDGE && (c & kClsFrozen) && !(from_s && s == 1)) close();
+      } else if (EDGE && c) {
+        if (c & kClsSlow) {
+          // every own-node value is read at once and the bouncing ones kept:
+          // one LDS round trip instead of one per bouncing direction
+          float own_f[L::Q];
+          static_for<L::Q>([&](auto qc) {
+            constexpr int q = decltype(qc)::value;
+            if constexpr (q > 0) own_f[q] = tb_get<St, L, L::opp[q]>(sh.f[src][L::opp[q]][cell]);
+          });
+          if (moving) {
+            TileArgs* p = opaque_args(ap);
+            const float uw[3] = {p->uw[0], p->uw[1], p->uw[2]};
+            static_for<L::Q>([&](auto qc) {
+              constexpr int q = decltype(qc)::value;
+              if constexpr (q > 0) {
+                const float ci_uw = static_cast<float>(L::cx[q]) * uw[0] + static_cast<float>(L::cy[q]) * uw[1] +
+                                    static_cast<float>(L::cz[q]) * uw[2];
+                const float v = own_f[q] + 2.0f * L::w[q] * 1.0f * 3.0f * ci_uw;
+                if (moving & (1u << q)) own_f[q] = v;
+              }
+            });
+          }
           static_for<L::Q>([&](auto qc) {
             constexpr int q = decltype(qc)::value;
             if constexpr (q > 0) {
-              const float ci_uw = static_cast<float>(L::cx[q]) * uw[0] + static_cast<float>(L::cy[q]) * uw[1] +
-                                  static_cast<float>(L::cz[q]) * uw[2];
-              const float v = own_f[q] + 2.0f * L::w[q] * 1.0f * 3.0f * ci_uw;
-              if (moving & (1u << q)) own_f[q] = v;
+              if (bm & (1u << q)) f[q] = own_f[q];
             }
           });
         }
-        static_for<L::Q>([&](auto qc) {
-          constexpr int q = decltype(qc)::value;
-          if constexpr (q > 0) {
-            if (bm & (1u << q)) f[q] = own_f[q];
-          }
-        });
-      }
-      // the closures, of solid nodes in the inlet and outlet rows too (form_s_at)
-      if (EDGE && c && formed) {
-        if (c & kClsInlet) {
-          if (noisy) u_edge = inlet_velocity(e, y, n, k);
-          close_inlet<L>(f, u_edge, e.uin_y);
-        }
-        if ((c & kClsOutlet) && e.outflow == 1) apply_zh_outflow_d2q9(e, f);
+        close();
       }
       if constexpr (THERMAL) {
         float g[D2Q5::Q];
