@@ -228,7 +228,12 @@ enum wake_field {
  * storage of f_q - w_q with FP32 arithmetic.  plane_pad < 0 picks the
  * default padding of the population plane stride. */
 /* Device bytes a domain of this shape allocates (with the temperature
- * populations if thermal != 0); host-only, for admission control. */
+ * populations if thermal != 0); host-only, for admission control.  On first
+ * use come on top: 4 Q bytes a node for f_src / f_dst reads and noise, 4
+ * bytes a node for moving walls, the analytics' 4 bytes a node each, and for
+ * forces in 2D (a probe, or batch members with forces) 4 bytes a node and up
+ * to 1.5 KB per node holding a link, the probe's bounded by the populations
+ * or 64 MB (without that memory single steps take the forces). */
 long long wake_domain_bytes_needed(int dim, int lattice, int nx, int ny, int nz, int storage, long long plane_pad,
                                    int thermal);
 int wake_domain_create(int dim, int lattice, int nx, int ny, int nz, float tau, int storage, long long plane_pad,

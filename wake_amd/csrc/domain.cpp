@@ -765,9 +765,9 @@ bool Domain::tile_kind() const {
 }
 
 bool Domain::tiles_pay(int storage, bool thermal, uint64_t nodes) {
-  // Measured, us a step of single launches / tiles: FP32 channels 4.4 / 1.7 at
-  // 240 x 80, 13.2 / 8.3 at 1500 x 403, 202 / 147 at 4096^2; FP32 temperature
-  // 6.1 / 2.1 at 240 x 80, 36 / 31 at 1536 x 1024, 341 / 326 at 4096^2.  With
+  // Measured, us a step of single launches / tiles without forces: FP32
+  // channels 4.6 / 1.8 at 240 x 80, 12.8 / 8.6 at 1500 x 403, 202 / 147 at
+  // 4096^2; FP32 temperature 6.0 / 2.2 at 240 x 80, 36 / 31 at 1536 x 1024, 341 / 326 at 4096^2.  With
   // 16-bit storage a single launch moves half the bytes, so the largest
   // domains do without: TRT channels 19.2 / 19.7 at 1536 x 1024, 151 / 153 at
   // 4096^2 (MRT 135 / 130); temperature 14.3 / 13.7 at 1024 x 512, 30 / 37 at

@@ -7,10 +7,10 @@ namespace wake_hip {
 // instructions a step.  Eight waves a SIMD (two 32 x 32 tiles a compute unit)
 // cap the scalar registers at 80: left alone the kernel takes 106, which
 // fits seven waves, so one tile -- the MRT + LES channel of 1500 x 403 nodes
-// then takes 10.7 us a step instead of 8.3.
-// At 1536 x 1024 nodes FP32: 144 G node-steps/s plain BGK, 91 G for the
-// channel (single-step launches: 70 G); at 240 x 80: 1.7 us a step, where a
-// single-step launch takes 4.4.
+// then takes 10.7 us a step instead of 8.3.  (Figures without forces.)
+// At 1536 x 1024 nodes FP32: 146 G node-steps/s plain BGK, 90 G for the
+// channel (single-step launches: 78 G and 76 G); TRT channel of 240 x 80:
+// 1.8 us a step, where a single-step launch takes 4.6.
 template <class St, int COLL, bool LES, bool THERMAL, bool FORCE, bool EDGES, int T, int W, int H>
 __global__ __launch_bounds__(W * H) __attribute__((amdgpu_waves_per_eu(!THERMAL && H == 32 ? 8 : 4))) void k_tile2d(const StepArgs a, const typename St::T* __restrict__ ain,
                                                   typename St::T* __restrict__ aout, const float* __restrict__ gin,
@@ -87,8 +87,8 @@ int compute_units() {
 }
 
 // The low tile owns half the nodes for 3/4 of the waves: worth it while there
-// is a compute unit for each tile (240 x 80 nodes, TRT channel: 1.69 us a
-// step against 2.07), not beyond (256 x 256: 2.47 against 2.23).
+// is a compute unit for each tile (240 x 80 nodes, TRT channel without
+// forces: 1.69 us a step against 2.07), not beyond (256 x 256: 2.47 against 2.23).
 bool low_tiles(const StepArgs& a) {
   const dim3 g = tiles_of<kTbSteps, kTileW, kTileLowH>(a.nx, a.ny);
   return static_cast<long long>(g.x) * g.y <= compute_units();
