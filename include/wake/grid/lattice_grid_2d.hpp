@@ -82,6 +82,7 @@ class LatticeGrid2D {
   void enable_force_history(real_t cx, real_t cy, real_t r_max);
   // Forces of steps *first_step .. current_step() (Fx, Fy, torque_z).
   std::vector<Vec3> force_history(uint64_t* first_step = nullptr) const;
+  // `steps` steps, one launch each; the device time in ms.
   float run(int steps, CollisionType collision = CollisionType::MRT, real_t gx = 0.0f, real_t gy = 0.0f,
             bool use_les = false, real_t smag_const = DEFAULT_SMAGORINSKY_CONSTANT);
   void check_finite() const;
