@@ -318,7 +318,6 @@ void Domain::set_populations(const float* f_ref) {
 // right after set_populations() with FP32 storage: no field of those planes
 // has been formed, and they are then the noisy ones.
 void Domain::add_noise(float amplitude, uint64_t seed) {
-  if (!planes_given_) ensure_device_fields();
   form_planes();
   const int slot = state_slot();
   const float* planes[27];
@@ -1062,13 +1061,26 @@ const float* Domain::uy() { return mirror(2); }
 const float* Domain::uz() { return mirror(3); }
 const float* Domain::speed() { return mirror(4); }
 
-// S_k in the reference layout (FP32 planes of N) in d_sout_.
+// S_k in the reference layout (FP32 planes of N) in d_sout_, and with it the
+// moments where they are not current: those of this S, also when a change of
+// the configuration rounds it to 16-bit storage later.  (Planes just given
+// have none yet; a temperature's moments come from its own read-back.)
 void Domain::form_planes() {
   sync_device_config();
   StepArgs a = args(false);
   a.s_out = planes_scratch();
+  const bool moments = !dfields_valid_ && !planes_given_;
+  if (moments && thermal_) ensure_device_fields();
+  if (moments && !thermal_) {
+    a.rho = d_rho_;
+    a.ux = d_ux_;
+    a.uy = d_uy_;
+    a.uz = d_uz_;
+    a.speed = d_speed_;
+  }
   const bool from_s = s_buf_ >= 0;
   check(launch_readback(lattice_, storage_, from_s, a, buf_[from_s ? s_buf_ : a_buf_], stream_), "readback");
+  if (moments) dfields_valid_ = true;
   sout_is_fsrc_ = false;
 }
 
