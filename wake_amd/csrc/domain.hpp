@@ -376,6 +376,7 @@ class Domain {
   int n_fnodes_ = 0;
   uint64_t tile_first_ = 0, tile_end_ = 0;
   bool tile_lists_ = false;  // they are there for tile_epoch_ (or not needed: no links)
+  bool lists_built_ = false;  // once in this domain's life
   static constexpr int kListSteps = 24;
   uint64_t wait_epoch_ = ~0ull;  // steps taken without them at this epoch
   int wait_steps_ = 0;
