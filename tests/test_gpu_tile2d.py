@@ -415,3 +415,35 @@ def test_batch_tiles_of_cavities(wa, sizes, coll, storage):
         ends.append([v for g in grids for v in _state(g, True)])
     for a, c in zip(*ends):
         assert np.array_equal(a, c, equal_nan=True)
+
+
+@pytest.mark.parametrize("storage", [0, 1, 2])
+def test_solid_nodes_on_open_boundaries_between_calls(wa, storage):
+    """f_dst after a change of the geometry, after one step from a given state
+    (which closes nothing) and after a batch."""
+    ends = []
+    for multi in (True, False):
+        g = _thick_channel(wa, 64, 33, storage, turb=True)
+        g.set_multistep(multi)
+        out = []
+        for steps in (9, 2, 16):
+            g.run(steps, "TRT")
+            g.set_cell_type(0, 30, 0)
+            g.set_cell_type(0, 29, 1)
+            out.append(g.f_dst_data().copy())
+            g.run(1, "TRT")
+            out.append(g.f_dst_data().copy())
+            g.set_populations(1.01 * g.f_src_data())
+            g.run(1, "TRT")
+            out.append(g.f_dst_data().copy())
+            g.run(2, "TRT")
+            out.append(g.f_dst_data().copy())
+            b = wa.Batch(lattice=9, storage=storage, collision="TRT", use_les=True, chunk=5)
+            slot = b.add(g, steps, smag=0.17)
+            b.run(steps)
+            b.remove(slot)
+            out.append(g.f_dst_data().copy())
+            out.append(g.f_src_data().copy())
+        ends.append(out)
+    for k, (a, b) in enumerate(zip(*ends)):
+        assert np.array_equal(a, b), k

@@ -216,6 +216,7 @@ void Domain::initialize(float rho, float ux, float uy, float uz) {
   upload_prev([&](size_t, int q) { return fe_q[q]; });
   s_buf_ = slot;
   a_buf_ = -1;
+  unclosed_ = false;
   std::fill(flags_.begin(), flags_.end(), static_cast<uint8_t>(kFluid));
   moving_cells_ = false;
   flags_dirty_ = cls_dirty_ = true;
@@ -253,6 +254,7 @@ void Domain::state_set(int slot) {
   clear_nonfinite();
   s_buf_ = slot;
   a_buf_ = -1;
+  unclosed_ = false;
   fsrc_valid_ = fdst_valid_ = sout_is_fsrc_ = false;
   if (probe_) probe_restart();  // the state the samples were taken of is gone
 }
@@ -738,8 +740,19 @@ void Domain::sync_device_config() {
   }
 }
 
+// Solid nodes in the inlet and outlet rows as single steps leave them.
+void Domain::close_solids() {
+  if (unclosed_ && dim_ == 2 && (has_inflow_ || outflow_ == 1)) {
+    StepArgs a = args(false);
+    a.s_step = step_count_ - 1;
+    check(launch_close_solid(storage_, a, buf_[a_buf_], stream_), "solid nodes");
+  }
+  unclosed_ = false;
+}
+
 void Domain::materialize() {
   sync_device_config();
+  close_solids();  // f_dst may be read after the change this comes before
   if (probe_) {
     // the force sample of S_k is taken from the unrounded S, as a pull
     // launch would take it, before the state is stored
@@ -813,6 +826,7 @@ void Domain::step_tile(int nsteps, int collision, float gx, float gy, bool use_l
         "tile steps");
   a_buf_ = out;
   s_buf_ = -1;
+  unclosed_ = nsteps > (from_s ? 1 : 0);
   g_last_[0] = gx;
   g_last_[1] = gy;
   g_last_[2] = 0.0f;
@@ -889,6 +903,7 @@ void Domain::step(int collision, float gx, float gy, float gz, bool use_les, flo
   g_last_[0] = gx;
   g_last_[1] = gy;
   g_last_[2] = gz;
+  unclosed_ = false;
   ++step_count_;
   invalidate_mirrors();
 }
@@ -1109,6 +1124,7 @@ void Domain::read_f_src(float* out) {
 // the initial state.
 bool Domain::form_dst_planes() {
   if (a_buf_ < 0) return false;
+  close_solids();
   StepArgs a = args(false);
   a.s_out = planes_scratch();
   // planes only: read the buffer as-is (no moments written)
@@ -1574,6 +1590,7 @@ void Domain::batch_prepare(float gx, float gy, float gz, float smag, StepArgs& a
 
 void Domain::batch_advance(uint64_t k, int parity_after, float gx, float gy, float gz) {
   if (k == 0) return;
+  unclosed_ = k > (s_buf_ >= 0 ? 1u : 0u);
   a_buf_ = parity_after;
   s_buf_ = -1;
   step_count_ += k;

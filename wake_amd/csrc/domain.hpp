@@ -238,6 +238,7 @@ class Domain {
   void refresh_mirrors(unsigned want);  // those of `want` and all handed out before
   void ensure_analytics(int which);     // device analytics arrays current
   bool form_dst_planes();               // A_{k-1} planes into d_sout_ (false: no step yet)
+  void close_solids();
   int state_slot();
   void state_set(int slot);
   void refresh_held();
@@ -332,6 +333,7 @@ class Domain {
   bool moving_cells_ = false;    // a cell was set to MovingWall since the last initialize()
   bool all_fluid_ = false;       // every cell type Fluid (set with the class bytes)
   void step_tile(int nsteps, int collision, float gx, float gy, bool use_les, float smag);
+  bool unclosed_ = false;        // steps since the state was set may have left solid open-boundary nodes unclosed
   bool tile_enabled_ = true;     // run() may take up to kTbSteps steps per launch
   int* d_aux_ = nullptr;
   BflNode* d_bfl_ = nullptr;

@@ -157,6 +157,9 @@ hipError_t launch_tile2d(int storage, int collision, bool les, bool thermal, boo
 // of mf.ring steps) of steps first .. first + count - 1 from those sums.
 hipError_t launch_mem_slots(const TileForces& mf, const int* row_list, int nrows, int nx, long long first, int count,
                             double* ring, hipStream_t s);
+// The closures of step a.s_step at the solid nodes of a 2D domain's inlet and
+// outlet rows, which tile launches leave out, in the populations buf.
+hipError_t launch_close_solid(int storage, const StepArgs& a, void* buf, hipStream_t s);
 // index[nodes[i]] = i.
 hipError_t launch_index_nodes(const int* nodes, int count, int* index, hipStream_t s);
 hipError_t launch_mark_bfl(const int* nodes, int count, uint8_t* cls, int* aux, hipStream_t s);

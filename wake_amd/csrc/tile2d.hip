@@ -58,6 +58,32 @@ __global__ __launch_bounds__(256) void k_mem_slots(const TileForces mf, const in
   }
 }
 
+// The open-boundary closures of step a.s_step at the solid nodes of the inlet
+// and outlet rows, in place in the populations that step left (form_s_at
+// applies them there each step).  Each forms three populations from six that
+// it leaves alone, so the last step's are all that is to be seen of them, and
+// closing again changes nothing.
+template <class St>
+__global__ __launch_bounds__(64) void k_close_solid(const StepArgs a, typename St::T* __restrict__ buf) {
+  using L = D2Q9;
+  const int y = blockIdx.x * 64 + threadIdx.x, x = blockIdx.y == 0 ? 0 : a.nx - 1;
+  if (y >= a.ny) return;
+  const int n = y * a.nx + x;
+  const uint8_t c = a.cls[n];
+  if (!(c & kClsFrozen)) return;
+  float f[L::Q];
+  static_for<L::Q>([&](auto qc) {
+    constexpr int q = decltype(qc)::value;
+    f[q] = tb_get<St, L, q>(buf[q * a.stride + n]);
+  });
+  if (c & kClsInlet) apply_inlet<L>(a, f, y, n, a.s_step);
+  if ((c & kClsOutlet) && a.outflow == 1) apply_zh_outflow_d2q9(a, f);
+  static_for<L::Q>([&](auto qc) {
+    constexpr int q = decltype(qc)::value;
+    buf[q * a.stride + n] = tb_put<St, L, q>(f[q]);
+  });
+}
+
 __global__ __launch_bounds__(256) void k_index_nodes(const int* __restrict__ nodes, int count,
                                                      int* __restrict__ index) {
   const int i = blockIdx.x * 256 + threadIdx.x;
@@ -188,6 +214,20 @@ hipError_t launch_mem_slots(const TileForces& mf, const int* row_list, int nrows
   if (nslots <= 0 || count <= 0) return hipSuccess;
   k_mem_slots<<<dim3((nslots + 3) / 4, count), 256, 0, s>>>(mf, row_list, waves, nslots, nx, first, ring);
   return hipGetLastError();
+}
+
+hipError_t launch_close_solid(int storage, const StepArgs& a, void* buf, hipStream_t s) {
+  auto with = [&](auto st) {
+    using St = decltype(st);
+    k_close_solid<St><<<dim3((a.ny + 63) / 64, 2), 64, 0, s>>>(a, static_cast<typename St::T*>(buf));
+    return hipGetLastError();
+  };
+  switch (storage) {
+    case kStoreF32: return with(StF32{});
+    case kStoreF16: return with(StF16{});
+    case kStoreBF16: return with(StBF16{});
+    default: return hipErrorInvalidValue;
+  }
 }
 
 hipError_t launch_index_nodes(const int* nodes, int count, int* index, hipStream_t s) {

@@ -17,9 +17,11 @@
 // has the same bits as that many single steps.  x always wraps; a tile row
 // outside a non-periodic y range holds wrapped values that no node inside
 // the range keeps (its bounce mask replaces them), as in the single-step
-// pull.  Not for curved links or the convective outlet (its upstream
-// neighbour reaches two nodes per step, past the halo): those domains take
-// single steps.
+// pull.  Solid nodes in the inlet and outlet rows are not closed here: no node
+// reads them, and k_close_solid does it before they are read out (tested for
+// in the step loop, they cost a batch of 512 wakes 1.2 %).  Not for curved
+// links or the convective outlet (its upstream neighbour reaches two nodes
+// per step, past the halo): those domains take single steps.
 #pragma once
 
 #include "thermal_impl.hpp"
@@ -204,13 +206,6 @@ __device__ __forceinline__ void tile2d_steps(Tile2dShared<St, THERMAL, W, H>& sh
       float f[L::Q];
       const bool pull = !(from_s && s == 1) && !(EDGE && (c & kClsFrozen));
       const unsigned long long k = s_step + static_cast<unsigned long long>(s - 1);  // S_k is formed here
-      auto close = [&]() {
-        if (c & kClsInlet) {
-          if (noisy) u_edge = inlet_velocity(e, y, n, k);
-          close_inlet<L>(f, u_edge, e.uin_y);
-        }
-        if ((c & kClsOutlet) && e.outflow == 1) apply_zh_outflow_d2q9(e, f);
-      };
       static_for<L::Q>([&](auto qc) {
         constexpr int q = decltype(qc)::value;
         f[q] = tb_get<St, L, q>(sh.f[src][q][cell - L::cy[q] * W - L::cx[q]]);
@@ -220,8 +215,6 @@ __device__ __forceinline__ void tile2d_steps(Tile2dShared<St, THERMAL, W, H>& sh
           constexpr int q = decltype(qc)::value;
           f[q] = tb_get<St, L, q>(sh.f[src][q][cell]);
         });
-        // solid nodes in the inlet and outlet rows are closed too, as form_s_at does
-        if (EDGE && (c & kClsFrozen) && !(from_s && s == 1)) close();
       } else if (EDGE && c) {
         if (c & kClsSlow) {
           // every own-node value is read at once and the bouncing ones kept:
@@ -251,7 +244,11 @@ __device__ __forceinline__ void tile2d_steps(Tile2dShared<St, THERMAL, W, H>& sh
             }
           });
         }
-        close();
+        if (c & kClsInlet) {
+          if (noisy) u_edge = inlet_velocity(e, y, n, k);
+          close_inlet<L>(f, u_edge, e.uin_y);
+        }
+        if ((c & kClsOutlet) && e.outflow == 1) apply_zh_outflow_d2q9(e, f);
       }
       if constexpr (THERMAL) {
         float g[D2Q5::Q];
