@@ -187,10 +187,10 @@ def batched_record(args):
     """Batched cylinder wakes: every domain stepped `steps` times by launches
     over all of them (several steps each where the domains allow it, else one
     with an autotuned shape; graph-captured chunks of 100), force history per
-    step, C_D and Strouhal per domain; the plain
-    one-domain-at-a-time path (the single-domain step with the same per-step
-    force, taken inside its step launch) is timed per domain on a short run
-    and scaled to the same step count.  Returns the record as a dict."""
+    step, C_D and Strouhal per domain; the plain one-domain-at-a-time path (the
+    same steps and per-step forces of one domain, taken inside its launches) is
+    timed per domain on a short run and scaled to the same step count.  Returns
+    the record as a dict."""
     import numpy as np
 
     import wake_amd
@@ -226,6 +226,7 @@ def batched_record(args):
     t0 = time.perf_counter()
     shape = b.tune(probe_steps=4)
     tune_s = time.perf_counter() - t0
+    b.run(4, use_graph=False)  # warm-up: the batch kernels' first launches
     left = max(b.remaining(s) for s in slots)
     log(f"single-step launch shape block={shape[0]} grid_factor={shape[1]} ({tune_s:.2f}s tuning; no effect on "
         f"launches of several steps); {left} steps left")
@@ -271,7 +272,7 @@ def batched_record(args):
             "batched_gbps": round(gbps, 1), "pull_d2q9_gbps": round(pull9, 1),
             "frac_of_pull_same_width": round(gbps / pull9, 4) if storage == 0 else None,
             "speedup_vs_plain": round(t_plain / t_batch, 3),
-            "plain": "single-domain step, one domain at a time, per-step force inside its step launch, wall time "
+            "plain": "one domain at a time, per-step force inside its step launches, wall time "
                      f"of a {probe}-step run per domain scaled to {S} steps",
             "error": "arithmetic identical to the plain path per node (bit-identical batch of one); members vs "
                      "the FP32 oracle within the FP32-floor criterion (tests/test_gpu_batch.py, test_gpu_configs.py)",
