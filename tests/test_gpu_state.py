@@ -260,7 +260,9 @@ def test_fields_go_with_the_populations_read(wa, lattice, shape, storage):
         g.set_inflow_west(0.04, 0.0)  # its nodes form values the storage does not hold
         g.run(3, "BGK", gx=1e-4, gy=2e-4)
         read(g)
+        f = g.f_src_data().copy()
         g.set_cell_type(*(3, 3, 3)[:2 if lattice == 9 else 3], 1)
+        assert np.array_equal(g.f_src_data(), f)  # as read before
         ends.append([g.rho_data(), g.ux_data(), g.uy_data(), g.speed_data()])
     for a, b in zip(*ends):
         assert np.array_equal(a, b)

@@ -1078,9 +1078,11 @@ const float* Domain::speed() { return mirror(4); }
 
 // S_k in the reference layout (FP32 planes of N) in d_sout_, and with it the
 // moments where they are not current: those of this S, also when a change of
-// the configuration rounds it to 16-bit storage later.  (Planes just given
-// have none yet; a temperature's moments come from its own read-back.)
+// the configuration rounds it to 16-bit storage later, and the planes read
+// again are then these too.  (Planes just given have no moments yet; a
+// temperature's come from its own read-back.)
 void Domain::form_planes() {
+  if (sout_is_fsrc_) return;
   sync_device_config();
   StepArgs a = args(false);
   a.s_out = planes_scratch();
@@ -1096,7 +1098,7 @@ void Domain::form_planes() {
   const bool from_s = s_buf_ >= 0;
   check(launch_readback(lattice_, storage_, from_s, a, buf_[from_s ? s_buf_ : a_buf_], stream_), "readback");
   if (moments) dfields_valid_ = true;
-  sout_is_fsrc_ = false;
+  sout_is_fsrc_ = true;
 }
 
 const float* Domain::f_src() {
@@ -1105,7 +1107,6 @@ const float* Domain::f_src() {
   h_fsrc_.resize(static_cast<size_t>(Q_) * N_);
   device_to_host(h_fsrc_.data(), d_sout_, h_fsrc_.size() * sizeof(float), stream_);
   fsrc_valid_ = true;
-  sout_is_fsrc_ = true;
   refresh_mirrors(0);
   return h_fsrc_.data();
 }

@@ -413,7 +413,7 @@ class Domain {
   unsigned held_ = 0;                 // bit k: h_field_[k] was handed out
   std::mutex mirror_mutex_;
   bool fsrc_valid_ = false, fdst_valid_ = false;
-  bool sout_is_fsrc_ = false;  // d_sout_ holds the bytes of the current f_src() mirror
+  bool sout_is_fsrc_ = false;  // d_sout_ holds the planes f_src() gives
   bool dfields_valid_ = false;  // device moment arrays current
   bool planes_given_ = false;   // FP32 planes were set and no step taken since
 };
